@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "gsvk_common.hpp"
+#include "gsvk_conv_group.hpp"
 
 namespace gsvk {
 namespace {
@@ -58,6 +59,7 @@ struct ConvArgs {
   void* y;
   long cin, cout, T, ldx, ldc, ldy;  // T: input columns
   int k, dil, pad, nch, opad;
+  int halo;  // staged columns past a tile: (k - 1) dil, or ceil(k / u) - 1
   int epi;
   float slope;
   bool vec;
@@ -65,6 +67,8 @@ struct ConvArgs {
   int up;     // 0: Conv1d; u: transposed convolution with stride u (phase r = blockIdx.z)
   long Tout;  // transposed: output columns T u
   int pad_t;  // transposed: (k - u) / 2
+  int kq, kr, pq, pr, er;  // transposed: k, pad_t and Tout - 1 + pad_t divided by u (block_map)
+  long eq;
   long xspan;  // time tiles per XCD (the grid's x extent / kXcds), 0: x index = time tile
 };
 
@@ -93,25 +97,26 @@ struct Map {
   const uint16_t* wp;
 };
 
-__device__ __forceinline__ long ceil_div(long a, long b) { return a >= 0 ? (a + b - 1) / b : -((-a) / b); }
-__device__ __forceinline__ long floor_div(long a, long b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
-
-__device__ __forceinline__ Map block_map(const ConvArgs& a) {
+// The phases' geometry without a division on the device (a 64-bit one costs a workgroup several
+// hundred cycles before its first load): with k = kq u + kr, pad_t = pq u + pr and
+// Tout - 1 + pad_t = eq u + er, all formed on the host, phase r < u has
+//   kn = kq + (r < kr), and the phases before it r kq + min(r, kr) taps;
+//   qlo = ceil((pad_t - r) / u) = pq + (pr > r), qhi = floor((Tout - 1 + pad_t - r) / u) =
+//   eq - (er < r).
+__device__ __forceinline__ Map block_map(const ConvArgs& a, int r) {
   Map m;
   if (!a.up) {
     m.kn = a.k, m.nq = a.T, m.xoff = -a.pad, m.ostr = 1, m.obase = 0, m.wp = a.wp;
     return m;
   }
-  const int u = a.up, r = blockIdx.z;
-  m.kn = (a.k - r + u - 1) / u;
-  size_t taps_before = 0;
-  for (int r2 = 0; r2 < r; ++r2) taps_before += static_cast<size_t>((a.k - r2 + u - 1) / u);
+  m.kn = a.kq + (r < a.kr ? 1 : 0);
+  const size_t taps_before = static_cast<size_t>(r * a.kq + min(r, a.kr));
   m.wp = a.wp + taps_before * a.nch * a.opad * kChunk;
-  const long qlo = ceil_div(a.pad_t - r, u), qhi = floor_div(a.Tout - 1 + a.pad_t - r, u);
+  const long qlo = a.pq + (a.pr > r ? 1 : 0), qhi = a.eq - (a.er < r ? 1 : 0);
   m.nq = qhi - qlo + 1;
   m.xoff = qlo - (m.kn - 1);
-  m.ostr = u;
-  m.obase = qlo * u + r - a.pad_t;
+  m.ostr = a.up;
+  m.obase = qlo * a.up + r - a.pad_t;
   return m;
 }
 
@@ -327,7 +332,7 @@ __attribute__((amdgpu_waves_per_eu(conv_waves_per_eu<XM>(FS)))) void conv1d_mfma
                : static_cast<long>(blockIdx.x)) *
       TT;
   const long o0 = static_cast<long>(blockIdx.y) * (FS * NO);
-  const Map m = block_map(a);
+  const Map m = block_map(a, blockIdx.z);
   if (t0 >= m.nq) return;  // a phase with fewer positions than the grid covers (whole workgroup)
 
   // ---- x chunk: global -> registers -> LDS ------------------------------------------------------
@@ -669,6 +674,280 @@ int launch_tiles(const ConvArgs& a, hipStream_t st) {
   return launch_status();
 }
 
+// ---- small grids: K split over the waves ---------------------------------------------------------
+//
+// A convolution over few columns (a streamed chunk of audio, the 384-channel stage, its upsampler,
+// conv_pre) launches fewer workgroups than the chip has CUs, and in conv1d_mfma each of them walks
+// all C_in x k of its products one refill at a time: every refill's weights come from L2 or the
+// MALL and are asked for one group of products (a few hundred cycles) earlier, so the workgroup
+// waits out most of a memory latency per group. Here the waves of a workgroup share one tile of
+// 16 NT columns x 16 NO output rows and split its (chunk, tap) units: wave w takes units w, w + KW,
+// ... The x tile of a batch of chunks is staged in LDS once, for all waves and taps; each wave reads
+// its units' weights straight from global memory into B fragments (no wave shares a unit, so there
+// is nothing to share through LDS), D units ahead, and no barrier falls between units. The
+// waves' partial sums meet in LDS and are added in wave order. The sum of an output is formed in
+// another order than conv1d_mfma's.
+struct KsArgs {
+  int tth;       // staged columns: 16 NT + halo, a multiple of 16
+  uint32_t tth_inv;  // ceil(2^32 / tth): mulhi(i, tth_inv) = i / tth for i < 2^16
+  int cb;        // chunks per batch
+  unsigned ntiles_t, ntiles_o, phases;
+  unsigned span;  // tiles per XCD
+  int esz_row;   // bytes of a row of x
+};
+
+template <int XM, int NT, int NO, int KW, int D>
+__device__ __forceinline__ void ksplit_tile(const ConvArgs& a, const KsArgs& ks, unsigned tile,
+                                            _Float16* xs) {
+  constexpr int DT = storage_dt<XM>();
+  constexpr int P = planes<XM>();
+  constexpr int TT = 16 * NT;
+  constexpr int TPB = kWave * KW;  // threads
+  constexpr int ESZ = DT == GSVK_F32 ? 4 : 2;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r16 = lane & 15, grp = lane >> 4;
+
+  // Tiles are numbered time fastest, then output-row blocks, then phases.
+  const unsigned oz = tile / ks.ntiles_t, z = oz / ks.ntiles_o;  // phase (0 without phases)
+  if (z >= ks.phases) return;
+  const Map m = block_map(a, static_cast<int>(z));
+  const long o0 = static_cast<long>(oz - z * ks.ntiles_o) * (16 * NO);
+  const long t0 = static_cast<long>(tile - oz * ks.ntiles_t) * TT;
+  if (t0 >= m.nq) return;
+
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(m.wp), 0, 0x7FFFFFFF, 0x00020000);
+  const int unit_bytes = static_cast<int>(a.opad) * 4 * 16;
+  int wofs[NO];
+#pragma unroll
+  for (int n = 0; n < NO; ++n)
+    wofs[n] = (grp * static_cast<int>(a.opad) + static_cast<int>(o0) + 16 * n + r16) * 16;
+  u32x4 wr[D][NO];
+  auto wload = [&](u32x4 (&w)[NO], int s) {
+#pragma unroll
+    for (int n = 0; n < NO; ++n)
+      w[n] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wofs[n], s * unit_bytes, 0);
+  };
+
+  f4v acc[NT][NO];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int n = 0; n < NO; ++n) acc[i][n] = f4v{0.f, 0.f, 0.f, 0.f};
+
+  // The epilogue's operands of the fragments this wave will finish: asked for first, used last.
+  constexpr int F = NT * NO;
+  constexpr int FPW = (F + KW - 1) / KW;  // fragments each wave finishes
+  const bool has_res = a.epi == GSVK_CONV_EPI_RES_LRELU || a.epi == GSVK_CONV_EPI_RES;
+  f4v cur[FPW];
+  float bias[FPW];
+#pragma unroll
+  for (int u = 0; u < FPW; ++u) {
+    const int f = min(wave + KW * u, F - 1);
+    const long o = o0 + 16 * (f % NO) + r16, t = t0 + 16 * (f / NO) + 4 * grp;
+    bias[u] = a.bias ? a.bias[min(o, a.cout - 1)] : 0.f;
+    if (has_res) cur[u] = load_cur<DT>(a, m, o, t);
+  }
+  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(a.x), 0,
+      static_cast<int>(a.cin - 1) * ks.esz_row + static_cast<int>(a.T) * ESZ, 0x00020000);
+  float m1 = -1.f;
+  asm("" : "+s"(m1));
+  const int tth = ks.tth;
+  const int actk = a.xact ? 1 : 0;
+  const int tbase = static_cast<int>(t0 + m.xoff);  // x column of staged column 0
+
+  for (int c0 = 0; c0 < a.nch; c0 += ks.cb) {
+    const int cn = min(ks.cb, a.nch - c0);
+    const int nu = cn * m.kn, u0 = c0 * m.kn;  // units of this batch
+    // the first D units' weights travel while x is staged
+#pragma unroll
+    for (int d = 0; d < D; ++d) wload(wr[d], u0 + min(wave + KW * d, nu - 1));
+
+    // ---- x: chunks c0 .. c0 + cn - 1, columns t0 + xoff .. + tth - 1 ---------------------------
+    // Item = one 16-byte row of LDS: 8 channels of one column. Loads are at clamped columns and
+    // channels (always inside x), zeroed outside [0, T) and past C_in when they are staged.
+    const int items = cn * 4 * tth;
+    constexpr int U = 4;
+    for (int i0 = 0; i0 < items; i0 += TPB * U) {
+      uint32_t raw[U][8];
+      bool ok[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int it = min(i0 + tid + TPB * u, items - 1);
+        const int g = static_cast<int>(__umulhi(static_cast<uint32_t>(it), ks.tth_inv));  // it / tth
+        const int t = tbase + it - g * tth, ch = c0 * kChunk + 8 * g;
+        ok[u] = t >= 0 && t < static_cast<int>(a.T) && ch < static_cast<int>(a.cin);
+        const int off = min(ch, static_cast<int>(a.cin) - 8) * ks.esz_row +
+                        min(max(t, 0), static_cast<int>(a.T) - 1) * ESZ;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if constexpr (DT == GSVK_F32)
+            raw[u][j] = __builtin_amdgcn_raw_buffer_load_b32(xrs, off, j * ks.esz_row, 0);
+          else
+            raw[u][j] = __builtin_amdgcn_raw_buffer_load_b16(xrs, off, j * ks.esz_row, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int it = i0 + tid + TPB * u;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          v[j] = DT == GSVK_F32 ? __builtin_bit_cast(float, raw[u][j]) : h2f(raw[u][j]);
+          v[j] = ok[u] ? v[j] : 0.f;
+          if (actk) v[j] = lrelu_ref(v[j], a.slope);
+        }
+        if (it < items) {
+          if constexpr (P == 2) {
+            const u32x4 hi = {pack_h2(v[0], v[1]), pack_h2(v[2], v[3]), pack_h2(v[4], v[5]),
+                              pack_h2(v[6], v[7])};
+            const u32x4 lo = {split_rest2(hi[0], v[0], v[1], m1),
+                              split_rest2(hi[1], v[2], v[3], m1),
+                              split_rest2(hi[2], v[4], v[5], m1),
+                              split_rest2(hi[3], v[6], v[7], m1)};
+            *reinterpret_cast<u32x4*>(xs + static_cast<size_t>(it) * 8) = hi;
+            *reinterpret_cast<u32x4*>(xs + static_cast<size_t>(ks.cb * 4 * tth + it) * 8) = lo;
+          } else {
+            const u32x4 hi = {f2h2(v[0], v[1]), f2h2(v[2], v[3]), f2h2(v[4], v[5]),
+                              f2h2(v[6], v[7])};
+            *reinterpret_cast<u32x4*>(xs + static_cast<size_t>(it) * 8) = hi;
+          }
+        }
+      }
+    }
+    __syncthreads();
+
+    // ---- this wave's units ----------------------------------------------------------------------
+    int c = wave / m.kn, kk = wave - c * m.kn;  // chunk of the batch and tap of the next unit
+    for (int j0 = wave; j0 < nu; j0 += KW * D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        if (j0 + KW * d < nu) {
+          const _Float16* xw =
+              xs + (static_cast<size_t>(c * 4 + grp) * tth + r16 + kk * a.dil) * 8;
+          h8 xf[NT][P];
+#pragma unroll
+          for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+              xf[i][p] = *reinterpret_cast<const h8*>(
+                  xw + (static_cast<size_t>(p) * ks.cb * 4 * tth + 16 * i) * 8);
+#pragma unroll
+          for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int n = 0; n < NO; ++n)
+#pragma unroll
+              for (int i = 0; i < NT; ++i)
+                acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    xf[i][p], __builtin_bit_cast(h8, wr[d][n]), acc[i][n], 0, 0, 0);
+          kk += KW;
+          while (kk >= m.kn) kk -= m.kn, ++c;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        wload(wr[d], u0 + min(j0 + KW * (d + D), nu - 1));
+      }
+    }
+    __syncthreads();  // x and, after the last batch, the reduction area
+  }
+
+  // ---- sum over the waves, epilogue -------------------------------------------------------------
+  f4v* red = reinterpret_cast<f4v*>(xs);
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int n = 0; n < NO; ++n) red[(wave * F + i * NO + n) * kWave + lane] = acc[i][n];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < FPW; ++u) {
+    const int f = wave + KW * u;
+    if (F % KW != 0 && f >= F) break;
+    f4v sum = red[f * kWave + lane];
+#pragma unroll
+    for (int w = 1; w < KW; ++w) sum = sum + red[(w * F + f) * kWave + lane];
+    const long o = o0 + 16 * (f % NO) + r16, t = t0 + 16 * (f / NO) + 4 * grp;
+    if (o < a.cout && t < m.nq) finish4<DT>(a, m, o, t, sum, bias[u], cur[u]);
+  }
+}
+
+// Up to kConvGroupMax convolutions of one shape (the same C_in, C_out and T, their own taps,
+// dilations, weights and buffers) in one launch: the three ResBlocks of a decoder stage run their
+// m-th convolutions side by side without a stream or a graph branch for each.
+struct KsGroup {
+  ConvArgs a[kConvGroupMax];
+  KsArgs ks[kConvGroupMax];
+};
+
+// Workgroup id b runs on XCD b % kXcds and takes that XCD's tile b / kXcds: span consecutive tiles
+// of the first convolution, then of the next. One XCD's L2 then holds the weights of the few
+// output-row blocks (and phases) whose tiles it computes, instead of every XCD fetching all of them.
+template <int XM, int NT, int NO, int KW, int D, int W>
+__global__ __launch_bounds__(kWave * KW)
+__attribute__((amdgpu_waves_per_eu(W))) void conv1d_ksplit(KsGroup g) {
+  extern __shared__ __attribute__((aligned(16))) _Float16 xs[];
+  const unsigned xcd = blockIdx.x % kXcds, i = blockIdx.x / kXcds;
+  const unsigned span = g.ks[0].span, j = i / span;
+  ksplit_tile<XM, NT, NO, KW, D>(g.a[j], g.ks[j], xcd * span + (i - j * span), xs);
+}
+
+// LDS for x per workgroup: two workgroups of 8 waves share a CU's 160 KiB.
+constexpr int kKsLds = 64 * 1024;
+
+template <int XM, int NT, int NO, int KW, int D, int W>
+int launch_ksplit(const ConvArgs* a, int n, hipStream_t st) {
+  auto kern = conv1d_ksplit<XM, NT, NO, KW, D, W>;
+  KsGroup g{};
+  const long npos = a->up ? a->T + 1 : a->T;
+  size_t lds = static_cast<size_t>(KW) * NT * NO * kWave * 16;  // the partial sums
+  for (int j = 0; j < n; ++j) {
+    g.a[j] = a[j];
+    KsArgs& ks = g.ks[j];
+    ks.tth = (16 * NT + a[j].halo + 15) / 16 * 16;
+    ks.tth_inv = static_cast<uint32_t>(((1ull << 32) + ks.tth - 1) / ks.tth);
+    const int chunk_bytes = planes<XM>() * 4 * ks.tth * 16;
+    const int cb = std::max(1, kKsLds / chunk_bytes);
+    const int nb = (a->nch + cb - 1) / cb;
+    ks.cb = (a->nch + nb - 1) / nb;
+    lds = std::max(lds, static_cast<size_t>(ks.cb) * chunk_bytes);
+    ks.ntiles_t = static_cast<unsigned>((npos + 16 * NT - 1) / (16 * NT));
+    ks.ntiles_o = static_cast<unsigned>((a->cout + 16 * NO - 1) / (16 * NO));
+    ks.phases = static_cast<unsigned>(a->up ? a->up : 1);
+    ks.span = (ks.ntiles_t * ks.ntiles_o * ks.phases + kXcds - 1) / kXcds;
+    ks.esz_row = static_cast<int>(a[j].ldx) * (storage_dt<XM>() == GSVK_F32 ? 4 : 2);
+  }
+  hipLaunchKernelGGL(kern, dim3(g.ks[0].span * kXcds * static_cast<unsigned>(n)), dim3(kWave * KW),
+                     lds, st, g);
+  return launch_status();
+}
+
+// 64 x 32 tiles of a convolution, all phases.
+long ks_tiles(const ConvArgs& a) {
+  return ((a.up ? a.T + 1 : a.T) + 63) / 64 * ((a.cout + 31) / 32) * (a.up ? a.up : 1);
+}
+
+// Whether conv1d_ksplit can run a: its staging loads eight channels of one column at 32-bit offsets
+// into the whole of x.
+bool ks_ok(const ConvArgs& a, size_t esz) {
+  return a.halo <= 64 && a.cout >= 24 && a.cin % 8 == 0 &&
+         static_cast<size_t>(a.cin) * a.ldx * esz < (1ul << 31);
+}
+
+// Tiles: 64 columns x 32 rows with 8 waves while all tiles of the launch run at once (two
+// workgroups per CU) and there are three units for every wave; otherwise 4 waves, on 48 rows with
+// the exact split (whose staging is twice as long) where that pads nothing.
+template <int XM>
+int launch_ks(const ConvArgs* a, int n, hipStream_t st) {
+  const int kn = (a->k + (a->up ? a->up : 1) - 1) / (a->up ? a->up : 1);
+  if (n * ks_tiles(*a) <= 600 && a->nch * kn >= 24)
+    return launch_ksplit<XM, 4, 2, 8, 4, 4>(a, n, st);
+  if constexpr (XM == kXSplit) {
+    if (a->cout >= 96 && a->cout % 48 == 0) return launch_ksplit<XM, 4, 3, 4, 4, 3>(a, n, st);
+  }
+  return launch_ksplit<XM, 4, 2, 4, 2, 4>(a, n, st);
+}
+
 template <int XM, int NT, int HMAX>
 int launch_no(const ConvArgs& a, int no, hipStream_t st) {
   switch (no) {
@@ -698,7 +977,12 @@ int launch_plan(const ConvArgs& a, hipStream_t st) {
   // Halos of up to 16 columns (k 3 at dilations up to 8, every dilation-1 ResBlock convolution,
   // the upsamplers) take the kernels with the 16-column halo slab; measured on the decoder
   // graph, 3% faster exact than staging a 64-column halo block for them.
-  const int halo = a.up ? (a.k + a.up - 1) / a.up - 1 : (a.k - 1) * a.dil;
+  const int halo = a.halo;
+  // Few tiles: the K-split kernel. The line was measured on the whole decoder, its ResBlocks on
+  // concurrent branches, at 20 to 500 frames.
+  constexpr long kKsTiles = XM == kXSplit ? 600 : 800;
+  if (ks_ok(a, storage_dt<XM>() == GSVK_F32 ? 4 : 2) && ks_tiles(a) < kKsTiles)
+    return launch_ks<XM>(&a, 1, st);
   if (halo <= 64 && a.cout >= 24) {
     // 32-wide fragments, 64 positions x 64 output rows per wave (256 x 64 per workgroup), when
     // 64-row tiles pad at most a sixth of the rows and the grid still holds about 1.5 workgroups
@@ -767,9 +1051,9 @@ extern "C" int gsvk_conv1d_pack(const uint16_t* w, size_t c_out, size_t c_in, si
 namespace gsvk {
 namespace {
 
-// Validation and launch shared by both entry points. T: input columns; Tout: output columns.
-int conv_entry(ConvArgs a, int dtype, int round_x, size_t T, size_t Tout, size_t wb,
-               hipStream_t st) {
+// Validation shared by the entry points; fills in what depends on it. T: input columns; Tout: output
+// columns; wb: bytes of the packed weights.
+int conv_check(ConvArgs& a, int dtype, size_t T, size_t Tout, size_t wb) {
   if (dtype != GSVK_F32 && dtype != GSVK_F16) return GSVK_E_DTYPE;
   a.xact = (a.epi & GSVK_CONV_X_LRELU) != 0;
   a.epi &= ~GSVK_CONV_X_LRELU;
@@ -804,8 +1088,36 @@ int conv_entry(ConvArgs a, int dtype, int round_x, size_t T, size_t Tout, size_t
           (!a.cur || (ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a.cur) % va == 0)) &&
           (!a.res || reinterpret_cast<uintptr_t>(a.res) % va == 0);
   if (a.up && a.up != 1) a.vec = false;  // interleaved phases: element stores
+  return GSVK_OK;
+}
+
+int conv_entry(ConvArgs a, int dtype, int round_x, size_t T, size_t Tout, size_t wb,
+               hipStream_t st) {
+  if (int rc = conv_check(a, dtype, T, Tout, wb)) return rc;
   if (dtype == GSVK_F16) return launch_plan<kXF16>(a, st);
   return round_x ? launch_plan<kXRound>(a, st) : launch_plan<kXSplit>(a, st);
+}
+
+// Operands of a Conv1d whose sizes are in range (GSVK_E_SIZE / E_ARG otherwise).
+int conv1d_args(ConvArgs& a, const void* x, size_t ldx, const uint16_t* w_packed, const float* bias,
+                int epi, float slope, void* cur, const void* res, size_t ldc, void* y, size_t ldy,
+                size_t c_in, size_t c_out, size_t T, size_t k, size_t dilation) {
+  if (!c_in || !c_out || !T || !k || !dilation) return GSVK_E_SIZE;
+  if (c_in > (1ul << 24) || c_out > (1ul << 24) || k > 4096 || dilation > 4096 ||
+      T > (1ul << 31) - 512 || ldx > (1ul << 40) || ldy > (1ul << 40) || ldc > (1ul << 40))
+    return GSVK_E_SIZE;
+  if ((k - 1) * dilation > static_cast<size_t>(kMaxHalo)) return GSVK_E_ARG;
+  a = ConvArgs{};
+  a.x = x, a.wp = w_packed, a.bias = bias, a.cur = cur, a.res = res, a.y = y;
+  a.cin = static_cast<long>(c_in), a.cout = static_cast<long>(c_out), a.T = static_cast<long>(T);
+  a.ldx = static_cast<long>(ldx), a.ldc = static_cast<long>(ldc), a.ldy = static_cast<long>(ldy);
+  a.k = static_cast<int>(k), a.dil = static_cast<int>(dilation);
+  a.pad = static_cast<int>((k - 1) * dilation / 2);
+  a.nch = static_cast<int>((c_in + kChunk - 1) / kChunk);
+  a.opad = static_cast<int>((c_out + kOPad - 1) / kOPad * kOPad);
+  a.halo = static_cast<int>((k - 1) * dilation);
+  a.epi = epi, a.slope = slope;
+  return GSVK_OK;
 }
 
 }  // namespace
@@ -816,23 +1128,46 @@ extern "C" int gsvk_conv1d(int dtype, int round_x, const void* x, size_t ldx,
                            void* cur, const void* res, size_t ldc, void* y, size_t ldy,
                            size_t c_in, size_t c_out, size_t T, size_t k, size_t dilation,
                            void* stream) {
-  if (!c_in || !c_out || !T || !k || !dilation) return GSVK_E_SIZE;
-  if (c_in > (1ul << 24) || c_out > (1ul << 24) || k > 4096 || dilation > 4096 ||
-      T > (1ul << 31) - 512 || ldx > (1ul << 40) || ldy > (1ul << 40) || ldc > (1ul << 40))
-    return GSVK_E_SIZE;
-  if ((k - 1) * dilation > static_cast<size_t>(kMaxHalo)) return GSVK_E_ARG;
-  ConvArgs a{};
-  a.x = x, a.wp = w_packed, a.bias = bias, a.cur = cur, a.res = res, a.y = y;
-  a.cin = static_cast<long>(c_in), a.cout = static_cast<long>(c_out), a.T = static_cast<long>(T);
-  a.ldx = static_cast<long>(ldx), a.ldc = static_cast<long>(ldc), a.ldy = static_cast<long>(ldy);
-  a.k = static_cast<int>(k), a.dil = static_cast<int>(dilation);
-  a.pad = static_cast<int>((k - 1) * dilation / 2);
-  a.nch = static_cast<int>((c_in + kChunk - 1) / kChunk);
-  a.opad = static_cast<int>((c_out + kOPad - 1) / kOPad * kOPad);
-  a.epi = epi, a.slope = slope;
+  ConvArgs a;
+  if (int rc = conv1d_args(a, x, ldx, w_packed, bias, epi, slope, cur, res, ldc, y, ldy, c_in,
+                           c_out, T, k, dilation))
+    return rc;
   return conv_entry(a, dtype, round_x, T, T, gsvk_conv1d_packed_elems(c_out, c_in, k) * 2,
                     static_cast<hipStream_t>(stream));
 }
+
+namespace gsvk {
+
+bool conv1d_group_pays(size_t C, size_t T) { return (T + 63) / 64 * ((C + 31) / 32) <= 200; }
+
+int conv1d_group(int dtype, int round_x, const ConvItem* items, int n, int epi, float slope,
+                 size_t ld, size_t C, size_t T, void* stream) {
+  if (n < 1 || n > kConvGroupMax) return GSVK_E_SIZE;
+  ConvArgs a[kConvGroupMax];
+  bool one = n > 1;  // every convolution can run in the one launch
+  for (int j = 0; j < n; ++j) {
+    const ConvItem& it = items[j];
+    if (int rc = conv1d_args(a[j], it.x, ld, it.w_packed, it.bias, epi, slope, it.cur, it.res, ld,
+                             it.y, ld, C, C, T, it.k, it.dilation))
+      return rc;
+    if (int rc = conv_check(a[j], dtype, T, T, gsvk_conv1d_packed_elems(C, C, it.k) * 2)) return rc;
+    one = one && ks_ok(a[j], dtype_size(dtype));
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (one) {
+    if (dtype == GSVK_F16) return launch_ks<kXF16>(a, n, st);
+    return round_x ? launch_ks<kXRound>(a, n, st) : launch_ks<kXSplit>(a, n, st);
+  }
+  for (int j = 0; j < n; ++j) {
+    int rc = dtype == GSVK_F16 ? launch_plan<kXF16>(a[j], st)
+             : round_x         ? launch_plan<kXRound>(a[j], st)
+                               : launch_plan<kXSplit>(a[j], st);
+    if (rc) return rc;
+  }
+  return GSVK_OK;
+}
+
+}  // namespace gsvk
 
 extern "C" size_t gsvk_convt1d_packed_elems(size_t c_out, size_t c_in, size_t k, size_t stride) {
   if (!c_out || !c_in || !k || !stride || k < stride) return 0;
@@ -880,9 +1215,13 @@ extern "C" int gsvk_convt1d(int dtype, int round_x, const void* x, size_t ldx,
   a.k = static_cast<int>(k), a.dil = 1, a.pad = 0;
   a.nch = static_cast<int>((c_in + kChunk - 1) / kChunk);
   a.opad = static_cast<int>((c_out + kOPad - 1) / kOPad * kOPad);
+  a.halo = static_cast<int>((k + stride - 1) / stride - 1);
   a.epi = epi, a.slope = slope;
   a.up = static_cast<int>(stride), a.Tout = static_cast<long>(T * stride);
   a.pad_t = static_cast<int>((k - stride) / 2);
+  a.kq = a.k / a.up, a.kr = a.k % a.up;
+  a.pq = a.pad_t / a.up, a.pr = a.pad_t % a.up;
+  a.eq = (a.Tout - 1 + a.pad_t) / a.up, a.er = static_cast<int>((a.Tout - 1 + a.pad_t) % a.up);
   return conv_entry(a, dtype, round_x, T, T * stride,
                     gsvk_convt1d_packed_elems(c_out, c_in, k, stride) * 2,
                     static_cast<hipStream_t>(stream));

@@ -1,0 +1,40 @@
+// gsvk_conv_group.hpp — several same-shape convolutions in one launch (internal to the library).
+#ifndef GSVK_CONV_GROUP_HPP
+#define GSVK_CONV_GROUP_HPP
+
+#include <cstddef>
+#include <cstdint>
+
+namespace gsvk {
+
+constexpr int kConvGroupMax = 3;
+
+// One convolution of a group: gsvk_conv1d's operands of that name (rows of stride ld).
+struct ConvItem {
+  const void* x;
+  const uint16_t* w_packed;
+  const float* bias;
+  void* cur;
+  const void* res;
+  void* y;
+  size_t k, dilation;
+};
+
+// Whether running a decoder stage's three convolutions as one launch beats three concurrent
+// branches: up to 200 tiles of 64 columns x 32 rows each, i.e. while the three fit the chip in about
+// one round. Measured on the whole decoder (fp16 storage / exact fp32): 20 frames 434 -> 368 and
+// 495 -> 459 us; every stage grouped at 150 frames 834 -> 935 and 1086 -> 1194, since a branch runs
+// into the next convolution while another's last workgroups drain and a group cannot.
+bool conv1d_group_pays(size_t C, size_t T);
+
+// n (1 .. kConvGroupMax) convolutions C -> C over T columns, each as gsvk_conv1d(dtype, round_x, x,
+// ld, w_packed, bias, epi, slope, cur, res, ld, y, ld, C, C, T, k, dilation, stream), in one launch
+// where the kernel for few tiles can run them all, otherwise one after another.
+// No convolution may read what another of the group writes. List the longest (largest k) first: its
+// workgroups start first.
+int conv1d_group(int dtype, int round_x, const ConvItem* items, int n, int epi, float slope,
+                 size_t ld, size_t C, size_t T, void* stream);
+
+}  // namespace gsvk
+
+#endif

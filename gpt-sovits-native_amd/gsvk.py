@@ -85,6 +85,8 @@ SIGNATURES = {
     "gsvk_sovits_decoder_workspace_bytes": (_sz, [_vp]),
     "gsvk_sovits_decoder_eager": (_i, [_vp, _vp]),
     "gsvk_sovits_decoder_create": (_i, [_vp, ctypes.POINTER(_vp)]),
+    "gsvk_sovits_stage_eager": (_i, [_i, _i, _vp, _vp, _sz, _sz, _f, _vp, _vp, _sz, _vp, _vp]),
+    "gsvk_sovits_stage_workspace_bytes": (_sz, [_i, _vp, _sz]),
 }
 
 
@@ -134,9 +136,20 @@ def _check(fn, rc):
     return rc
 
 
+class _DtypeCodes(dict):
+    def __missing__(self, dtype):
+        import torch
+        self.update({torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16})
+        if dtype not in self:
+            raise KeyError(dtype)
+        return self[dtype]
+
+
+_DTYPE = _DtypeCodes()
+
+
 def dtype_code(t):
-    import torch
-    return {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}[t.dtype]
+    return _DTYPE[t.dtype]
 
 
 def _rows(t):
@@ -314,9 +327,11 @@ class GeneratorStage:
                                                   no copy of y
       out = lrelu(mean_j cur_j, slope_next)       mul_write / add_scaled_inplace + the next stage's
                                                   leaky_relu_io (dec.hpp:328-336, 284 or 342)
-    Launches: 1 upsampler, 18 convolutions, 1 branch mean. ResBlocks after the first run on side
-    streams of their own (each with its own t_a), forked after the upsampler and joined back before
-    the branch mean, as in gsvk_sovits_decoder_*."""
+    20 passes: 1 upsampler, 18 convolutions, 1 branch mean, issued by gsvk_sovits_stage_eager as the
+    decoder issues them: the ResBlocks' m-th convolutions as one launch where the stage has few
+    columns, otherwise ResBlocks beside each other on two side streams of this object, joined back
+    before the branch mean. Stages of another make-up than three ResBlock1s of three pairs, all of
+    one channel count and the same dilations, are issued pass by pass."""
 
     def __init__(self, ups, resblocks):
         self.ups = ups
@@ -332,6 +347,14 @@ class GeneratorStage:
             self._buf = (key, mk(), [mk() for _ in self.resblocks], [mk() for _ in self.resblocks])
         return self._buf[1:]
 
+    def _workspace(self, S, T, dtype, device):
+        import torch
+        need = lib().gsvk_sovits_stage_workspace_bytes(_DTYPE[dtype], S, T)
+        key = (need, device)
+        if need and (self._buf is None or self._buf[0] != key):
+            self._buf = (key, torch.empty(need, dtype=torch.uint8, device=device))
+        return (self._buf[1].data_ptr(), need) if need else (None, 0)
+
     def _side_streams(self, device):
         import torch
         if self._side is None or self._side[0] != device:
@@ -339,13 +362,48 @@ class GeneratorStage:
                                    for _ in self.resblocks[1:]])
         return self._side[1]
 
+    def _stage(self):
+        """The gsvk_sovits_stage of the weights as they are now (words in the struct's order), or None
+        where the stage is not of its make-up."""
+        ups, rbs = self.ups, self.resblocks
+        C = ups.out_c
+        if len(rbs) != 3:
+            return None
+        dil = [c.dilation for c in rbs[0].convs1]
+        for rb in rbs:
+            k = rb.convs1[0].k if rb.convs1 else 0
+            if (len(rb.convs1) != 3 or len(rb.convs2) != 3
+                    or [c.dilation for c in rb.convs1] != dil
+                    or any(c.dilation != 1 for c in rb.convs2)
+                    or any(c.k != k or c.in_c != C or c.out_c != C
+                           for c in rb.convs1 + rb.convs2)):
+                return None
+        w = [ups.in_c, C, ups.k, ups.stride_u, _ptr(ups.wp), _ptr(ups.b) or 0]
+        w += [rb.convs1[0].k for rb in rbs] + dil
+        w += [_ptr(c.wp) for rb in rbs for c in rb.convs1]
+        w += [_ptr(c.b) or 0 for rb in rbs for c in rb.convs1]
+        w += [_ptr(c.wp) for rb in rbs for c in rb.convs2]
+        w += [_ptr(c.b) or 0 for rb in rbs for c in rb.convs2]
+        return (ctypes.c_uint64 * 48)(*w)
+
     def forward(self, x, out, slope_next=0.1, round_x=False, stream=None):
         import torch
-        y, tas, curs = self._buffers(self.ups.out_c, x.shape[1] * self.ups.stride_u, x.dtype,
-                                     x.device)
         main = stream if stream is not None else torch.cuda.current_stream(x.device)
+        S = self._stage()
+        c_in, T, ldx = _rows(x)
+        if (S is not None and c_in == self.ups.in_c and out.dtype == x.dtype
+                and out.numel() == self.ups.out_c * T * self.ups.stride_u):
+            ws, need = self._workspace(S, T, x.dtype, x.device)
+            side = (_vp * 2)(*[s.cuda_stream for s in self._side_streams(x.device)])
+            _check("gsvk_sovits_stage_eager",
+                   lib().gsvk_sovits_stage_eager(_DTYPE[x.dtype], int(round_x), S, _ptr(x), ldx, T,
+                                                 slope_next, _ptr(out), ws, need, side,
+                                                 _stream(main)))
+            return out
         if isinstance(main, int):
             main = torch.cuda.ExternalStream(main, device=x.device)
+        y, tas, curs = self._buffers(self.ups.out_c, x.shape[1] * self.ups.stride_u, x.dtype,
+                                     x.device)
         self.ups.forward(x, y, round_x=round_x, stream=main)
         sides = self._side_streams(x.device)
         for sd in sides:

@@ -3,10 +3,12 @@
 // graph (gsvk_sovits_decoder_*).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 
 #include "gsvk.h"
+#include "gsvk_conv_group.hpp"
 #include "gsvk_sovits.h"
 
 namespace {
@@ -28,8 +30,8 @@ enum Slot {
   kSlots = kCur0 + GSVK_SOVITS_RESBLOCKS
 };
 
-// ResBlocks 1 and 2 of every stage run on two more streams, concurrent with ResBlock 0 on the main
-// one (they share only the upsampler's output, which they read); the branch mean waits for all
+// Where one launch for the three ResBlocks' m-th convolutions does not pay (conv1d_group_pays),
+// two of them run on two more streams, concurrent with the first on the main one (they share only the upsampler's output, which they read); the branch mean waits for all
 // three. In a recorded graph the streams and events are the capture's; eagerly, the side streams
 // are the device's own (below) and the events the call's.
 constexpr int kSide = GSVK_SOVITS_RESBLOCKS - 1;
@@ -96,9 +98,81 @@ int check_workspace(const gsvk_sovits_decoder_desc* d, Layout* lay) {
   return GSVK_OK;
 }
 
+// The passes of the decoder; three convolutions grouped into one launch count as three.
 int count_launches(const gsvk_sovits_decoder_desc* d) {
   // cond with the bias fold (with conditioning), conv_pre, 20 per stage, conv_post
   return (d->g_in ? 1 : 0) + 1 + 20 * static_cast<int>(d->n_stages) + 1;
+}
+
+// One Generator stage (dec.hpp:283-336): out = lrelu(mean_j ResBlock_j(ups(x)), slope_next). x
+// [c_in, T] with row stride ldx arrives LeakyReLU'd; buf[kY .. kSlots - 1] hold c_out x T ups_u
+// elements each. br: the streams ResBlocks 1 and 2 may run on (nullptr: all on st).
+int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_t ldx, size_t T,
+                void* const* buf, float slope_next, void* out, void* st, const Branches* br) {
+  const float slope = 0.1f;  // LRELU_SLOPE (dec.hpp:284, 322, 324)
+  const size_t C = S.c_out, Tu = T * S.ups_u;
+  // y = ups(x)  (dec.hpp:285)
+  if (int rc = gsvk_convt1d(dt, rx, x, ldx, S.ups_w, S.ups_b, GSVK_CONV_EPI_BIAS, 0.f, nullptr,
+                            nullptr, 0, buf[kY], Tu, S.c_in, C, T, S.ups_k, S.ups_u, st))
+    return rc;
+  T = Tu;
+  const void* curs[GSVK_SOVITS_RESBLOCKS];
+  gsvk::ConvItem c1[GSVK_SOVITS_PAIRS][GSVK_SOVITS_RESBLOCKS];
+  gsvk::ConvItem c2[GSVK_SOVITS_PAIRS][GSVK_SOVITS_RESBLOCKS];
+  size_t ord[GSVK_SOVITS_RESBLOCKS];  // ResBlocks, largest k first
+  for (size_t j = 0; j < GSVK_SOVITS_RESBLOCKS; ++j) ord[j] = j, curs[j] = buf[kCur0 + j];
+  std::sort(ord, ord + GSVK_SOVITS_RESBLOCKS,
+            [&](size_t p, size_t q) { return S.res_k[p] > S.res_k[q]; });
+  for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m)
+    for (size_t i = 0; i < GSVK_SOVITS_RESBLOCKS; ++i) {
+      const size_t j = ord[i];
+      void* cur = buf[kCur0 + j];
+      void* ta = buf[kTa0 + j];
+      // cur_j starts as a copy of y (dec.hpp:316): the first pair reads y in place
+      const void* src = m == 0 ? buf[kY] : cur;
+      // t_a = lrelu(convs1[m](lrelu(cur_j)))  (dec.hpp:322-324: leaky_relu_write as the
+      // convolution reads its input, leaky_relu_io in its store)
+      c1[m][i] = {src, S.w1[j][m], S.b1[j][m], nullptr, nullptr, ta, S.res_k[j], S.res_dil[m]};
+      // cur_j = res + convs2[m](t_a)  (dec.hpp:325-326)
+      c2[m][i] = {ta, S.w2[j][m], S.b2[j][m], cur, src, nullptr, S.res_k[j], 1};
+    }
+  // The convolutions of ResBlocks i .. i + n - 1 (in that order) on stream bst.
+  auto blocks = [&](size_t i, int n, void* bst) -> int {
+    for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m) {
+      if (int e = gsvk::conv1d_group(dt, rx, &c1[m][i], n,
+                                     GSVK_CONV_EPI_LRELU | GSVK_CONV_X_LRELU, slope, T, C, T,
+                                     bst))
+        return e;
+      if (int e = gsvk::conv1d_group(dt, rx, &c2[m][i], n, GSVK_CONV_EPI_RES, slope, T, C, T,
+                                     bst))
+        return e;
+    }
+    return GSVK_OK;
+  };
+  if (gsvk::conv1d_group_pays(C, T)) {
+    if (int rc = blocks(0, GSVK_SOVITS_RESBLOCKS, st)) return rc;
+  } else if (!br) {
+    for (size_t i = 0; i < GSVK_SOVITS_RESBLOCKS; ++i)
+      if (int rc = blocks(i, 1, st)) return rc;
+  } else {
+    int rc = GSVK_OK;  // (a failed wait still reaches the joins below)
+    if (hipEventRecord(br->fork, static_cast<hipStream_t>(st)) != hipSuccess) return GSVK_E_HIP;
+    for (int i = 0; i < kSide; ++i)
+      if (hipStreamWaitEvent(br->side[i], br->fork, 0) != hipSuccess) rc = GSVK_E_HIP;
+    for (size_t i = 0; i < GSVK_SOVITS_RESBLOCKS && rc == GSVK_OK; ++i)
+      rc = blocks(i, 1, i > 0 ? br->side[i - 1] : st);
+    // every side stream joins back, also after an error (a capture must end joined)
+    for (int i = 0; i < kSide; ++i)
+      if ((hipEventRecord(br->join[i], br->side[i]) != hipSuccess ||
+           hipStreamWaitEvent(static_cast<hipStream_t>(st), br->join[i], 0) != hipSuccess) &&
+          rc == GSVK_OK)
+        rc = GSVK_E_HIP;
+    if (rc) return rc;
+  }
+  // x = lrelu(mean_j cur_j): mul_write / add_scaled_inplace (dec.hpp:328-333) with the next
+  // stage's leaky_relu_io (dec.hpp:284, 0.1) or the final one (dec.hpp:342, 0.01).
+  return gsvk_resblock_branch_mean(dt, curs, nullptr, GSVK_SOVITS_RESBLOCKS, out, C * T, 1,
+                                   slope_next, st);
 }
 
 // The launches of one decoder pass in Generator::forward's order.
@@ -129,54 +203,10 @@ int issue(const gsvk_sovits_decoder_desc* d, const Layout& lay, void* st, const 
     return rc;
 
   for (size_t s = 0; s < d->n_stages; ++s) {
-    const gsvk_sovits_stage& S = d->stage[s];
-    const size_t C = S.c_out, Tu = T * S.ups_u;
-    // y = ups(x)  (dec.hpp:285)
-    if ((rc = gsvk_convt1d(dt, rx, slot[kX], T, S.ups_w, S.ups_b, GSVK_CONV_EPI_BIAS, 0.f, nullptr,
-                           nullptr, 0, slot[kY], Tu, S.c_in, C, T, S.ups_k, S.ups_u, st)))
-      return rc;
-    T = Tu;
-    if (br) {  // (a failed wait still reaches the joins below)
-      if (hipEventRecord(br->fork, static_cast<hipStream_t>(st)) != hipSuccess) return GSVK_E_HIP;
-      for (int i = 0; i < kSide; ++i)
-        if (hipStreamWaitEvent(br->side[i], br->fork, 0) != hipSuccess) rc = GSVK_E_HIP;
-    }
-    const void* curs[GSVK_SOVITS_RESBLOCKS];
-    for (size_t j = 0; j < GSVK_SOVITS_RESBLOCKS && rc == GSVK_OK; ++j) {
-      void* bst = br && j > 0 ? br->side[j - 1] : st;
-      void* cur = slot[kCur0 + j];
-      void* ta = slot[kTa0 + j];
-      curs[j] = cur;
-      const void* src = slot[kY];  // cur_j starts as a copy of y (dec.hpp:316): read it in place
-      const void* res = slot[kY];
-      for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m) {
-        // t_a = lrelu(convs1[m](lrelu(cur_j)))  (dec.hpp:322-324: leaky_relu_write as the
-        // convolution reads its input, leaky_relu_io in its store)
-        if ((rc = gsvk_conv1d(dt, rx, src, T, S.w1[j][m], S.b1[j][m],
-                              GSVK_CONV_EPI_LRELU | GSVK_CONV_X_LRELU, slope, nullptr, nullptr, 0,
-                              ta, T, C, C, T, S.res_k[j], S.res_dil[m], bst)))
-          break;
-        // cur_j = res + convs2[m](t_a)  (dec.hpp:325-326)
-        if ((rc = gsvk_conv1d(dt, rx, ta, T, S.w2[j][m], S.b2[j][m], GSVK_CONV_EPI_RES, slope, cur,
-                              res, T, nullptr, T, C, C, T, S.res_k[j], 1, bst)))
-          break;
-        src = cur;
-        res = nullptr;  // in place from the second pair on
-      }
-    }
-    if (br)  // every side stream joins back, also after an error (a capture must end joined)
-      for (int i = 0; i < kSide; ++i)
-        if ((hipEventRecord(br->join[i], br->side[i]) != hipSuccess ||
-             hipStreamWaitEvent(static_cast<hipStream_t>(st), br->join[i], 0) != hipSuccess) &&
-            rc == GSVK_OK)
-          rc = GSVK_E_HIP;
-    if (rc) return rc;
-    // x = lrelu(mean_j cur_j): mul_write / add_scaled_inplace (dec.hpp:328-333) with the next
-    // stage's leaky_relu_io (dec.hpp:284, 0.1) or the final one (dec.hpp:342, 0.01).
     const float next_slope = s + 1 < d->n_stages ? slope : 0.01f;
-    if ((rc = gsvk_resblock_branch_mean(dt, curs, nullptr, GSVK_SOVITS_RESBLOCKS, slot[kX], C * T,
-                                        1, next_slope, st)))
+    if ((rc = issue_stage(dt, rx, d->stage[s], slot[kX], T, T, slot, next_slope, slot[kX], st, br)))
       return rc;
+    T *= d->stage[s].ups_u;
   }
   // out = tanh(conv_post(x))  (dec.hpp:343-344; conv_post has no bias)
   return gsvk_conv1d(dt, rx, slot[kX], T, d->post_w, nullptr, GSVK_CONV_EPI_TANH, 0.f, nullptr,
@@ -215,6 +245,58 @@ __attribute__((visibility("hidden"))) int gsvk_record_graph_branches_(
 extern "C" size_t gsvk_sovits_decoder_workspace_bytes(const gsvk_sovits_decoder_desc* desc) {
   Layout lay;
   return shapes(desc, &lay) == GSVK_OK ? lay.bytes : 0;
+}
+
+// A stage alone: its shapes, and the bytes of one of its 7 buffers (0: invalid).
+static size_t stage_slot_bytes(int dtype, const gsvk_sovits_stage* S, size_t T) {
+  if (!S || (dtype != GSVK_F32 && dtype != GSVK_F16)) return 0;
+  if (T == 0 || S->c_in == 0 || S->c_out == 0 || S->ups_k == 0 || S->ups_u == 0) return 0;
+  for (size_t j = 0; j < GSVK_SOVITS_RESBLOCKS; ++j)
+    if (S->res_k[j] == 0) return 0;
+  for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m)
+    if (S->res_dil[m] == 0) return 0;
+  const size_t esz = dtype == GSVK_F32 ? 4 : 2;
+  if (T > SIZE_MAX / S->ups_u || T * S->ups_u > (SIZE_MAX / 2) / esz / kSlots / S->c_out) return 0;
+  return round_up(T * S->ups_u * S->c_out * esz, kAlign);
+}
+
+extern "C" size_t gsvk_sovits_stage_workspace_bytes(int dtype, const gsvk_sovits_stage* stage,
+                                                    size_t T) {
+  return (kSlots - kY) * stage_slot_bytes(dtype, stage, T);
+}
+
+extern "C" int gsvk_sovits_stage_eager(int dtype, int round_x, const gsvk_sovits_stage* stage,
+                                       const void* x, size_t ldx, size_t T, float slope_next,
+                                       void* out, void* workspace, size_t workspace_bytes,
+                                       void* const* side, void* stream) {
+  if (!stage || !x || !out || !workspace || !stage->ups_w) return GSVK_E_NULL;
+  for (size_t j = 0; j < GSVK_SOVITS_RESBLOCKS; ++j)
+    for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m)
+      if (!stage->w1[j][m] || !stage->w2[j][m]) return GSVK_E_NULL;
+  if (side && (!side[0] || !side[1])) return GSVK_E_NULL;
+  if (dtype != GSVK_F32 && dtype != GSVK_F16) return GSVK_E_DTYPE;
+  const size_t slot = stage_slot_bytes(dtype, stage, T);
+  if (slot == 0 || workspace_bytes < (kSlots - kY) * slot) return GSVK_E_SIZE;
+  if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return GSVK_E_ARG;
+  void* buf[kSlots] = {};
+  for (int i = kY; i < kSlots; ++i) buf[i] = static_cast<char*>(workspace) + (i - kY) * slot;
+  if (!side || gsvk::conv1d_group_pays(stage->c_out, T * stage->ups_u))
+    return issue_stage(dtype, round_x, *stage, x, ldx, T, buf, slope_next, out, stream, nullptr);
+  hipStream_t sd[kSide];
+  hipEvent_t fork = nullptr, join[kSide] = {};
+  int rc = hipEventCreateWithFlags(&fork, hipEventDisableTiming) == hipSuccess ? GSVK_OK : GSVK_E_HIP;
+  for (int i = 0; i < kSide && rc == GSVK_OK; ++i) {
+    sd[i] = static_cast<hipStream_t>(side[i]);
+    if (hipEventCreateWithFlags(&join[i], hipEventDisableTiming) != hipSuccess) rc = GSVK_E_HIP;
+  }
+  if (rc == GSVK_OK) {
+    const Branches br{sd, fork, join};
+    rc = issue_stage(dtype, round_x, *stage, x, ldx, T, buf, slope_next, out, stream, &br);
+  }
+  if (fork) (void)hipEventDestroy(fork);
+  for (int i = 0; i < kSide; ++i)
+    if (join[i]) (void)hipEventDestroy(join[i]);
+  return rc;
 }
 
 extern "C" int gsvk_sovits_decoder_eager(const gsvk_sovits_decoder_desc* desc, void* stream) {

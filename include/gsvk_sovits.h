@@ -8,7 +8,7 @@
  *                                            frame (gsvk_gemv_f16w), the broadcast add
  *                                            (dec.hpp:275-279) folded into its output
  *   x    = lrelu(conv_pre(z) + bias, 0.1)    (dec.hpp:268, 275-279, 284)          1 launch
- *   per stage s (dec.hpp:283-336):                                               20 launches
+ *   per stage s (dec.hpp:283-336):                        20 passes, 8 to 20 launches
  *     y = ups(x)
  *     per ResBlock j, pair m: t_a = lrelu(convs1[m](lrelu(c))), c = m ? cur_j : y   (X_LRELU input,
  *                             LRELU epilogue); cur_j = c + convs2[m](t_a)           (RES epilogue)
@@ -77,15 +77,28 @@ typedef struct gsvk_sovits_decoder_desc {
  * still be NULL); 0 on invalid shapes. Host only. */
 size_t gsvk_sovits_decoder_workspace_bytes(const gsvk_sovits_decoder_desc* desc);
 /* Issue the decoder's launches on `stream` (GSVK_E_NULL / E_SIZE / E_ARG on a bad descriptor).
- * ResBlocks 1 and 2 of each stage run on two streams the library keeps per device, ordered after
+ * Two ResBlocks of each stage run on two streams the library keeps per device, ordered after
  * the work already on `stream` and joined back into it (each stage's branch mean waits for them), so
- * `stream` orders the whole decoder as usual. Those streams are created on the device's first call:
+ * `stream` orders the whole decoder as usual; a stage of few columns (up to 200 tiles of 64 columns x
+ * 32 channels) runs the three ResBlocks' m-th convolutions as one launch on `stream` instead. Those streams are created on the device's first call:
  * a caller recording this call into a graph of its own makes one call outside the capture first
  * (gsvk_sovits_decoder_create records the same launches by itself). */
 int gsvk_sovits_decoder_eager(const gsvk_sovits_decoder_desc* desc, void* stream);
 /* Record the same launches into a HIP graph; run it with gsvk_t2s_step_run, free it with
- * gsvk_t2s_step_destroy. The graph keeps the descriptor's pointers: the buffers must outlive it. */
+ * gsvk_t2s_step_destroy (gsvk_t2s_step_launches counts its passes: 20 per stage however they are
+ * grouped). The graph keeps the descriptor's pointers: the buffers must outlive it. */
 int gsvk_sovits_decoder_create(const gsvk_sovits_decoder_desc* desc, gsvk_t2s_step** out);
+
+/* One Generator stage (dec.hpp:283-336) alone: out = lrelu(mean_j ResBlock_j(ups(x)), slope_next),
+ * with the launches the decoder issues for it. x [c_in, T] (row stride ldx >= T) arrives LeakyReLU'd;
+ * out [c_out, T * ups_u] contiguous; the workspace holds gsvk_sovits_stage_workspace_bytes bytes,
+ * 16-byte aligned. side: two streams of the caller's for ResBlocks that run beside each other, joined
+ * back into `stream` (a stage of few columns uses none), or NULL to keep everything on `stream`. */
+int gsvk_sovits_stage_eager(int dtype, int round_x, const gsvk_sovits_stage* stage, const void* x,
+                            size_t ldx, size_t T, float slope_next, void* out, void* workspace,
+                            size_t workspace_bytes, void* const* side, void* stream);
+/* 0 on invalid shapes. Host only. */
+size_t gsvk_sovits_stage_workspace_bytes(int dtype, const gsvk_sovits_stage* stage, size_t T);
 
 #ifdef __cplusplus
 }
