@@ -3,12 +3,15 @@
 // whole step with its GEMVs and attention (gsvk_t2s_decode_*).
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+#include <cstdint>
 #include <new>
 #include <type_traits>
 #include <vector>
 
 #include "gsvk.h"
 #include "gsvk_t2s.h"
+#include "gsvk_t2s_attn.hpp"
 
 namespace gsvk {
 // csrc/gsvk_step.hip: the device addresses the fused step's launch puts in place of absent
@@ -68,6 +71,59 @@ T* advance(T* p, size_t bytes) {
   return p ? reinterpret_cast<T*>(reinterpret_cast<B*>(p) + bytes) : nullptr;
 }
 
+// The batch in two parts. At decode sizes every launch but the attention scan is bound by latency,
+// not bandwidth, so the two parts' launch chains are recorded on two streams of one graph, which
+// the runtime issues on two hardware queues and runs side by side. Measured on the whole step
+// (B = 64, 24 layers): 1098 -> 1082-1092 us at 1024 cached keys and 1548-1555 -> 1457-1461 us at
+// 2048. The gain is small because one part's chain alone takes 916-1049 us: the chain's launch
+// latency, not its rows, sets the step time. Batches of fewer than kSplitRows sequences, and
+// workspaces too small for both parts' attention states, run as one part.
+constexpr size_t kSplitRows = 32;
+constexpr size_t kWsAlign = 256;
+
+// The fused launch reads W_qkv once per sequence and its keys in 64-byte pieces: it wins while few
+// keys are read in all. Whole step, us, separate launches against fused (csrc/gsvk_t2s_attn.hip): 1
+// sequence, 300 keys 631 -> 471; 8 x 1024 695 -> 647; 16 x 300 717 -> 549; 16 x 1088 732 -> 675;
+// 31 x 364 698 -> 670; 24 x 1088 797 -> 846.
+constexpr size_t kFusedKeys = 18000;
+
+bool overlap(const void* a, size_t an, const void* b, size_t bn) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+  return a && b && an && bn && p < q + bn && q < p + an;
+}
+
+// The one-launch form of layer l's QKV projection and attention (csrc/gsvk_t2s_attn.hip) for n rows
+// at those addresses, or false (and a null z) where the separate launches run.
+bool fused_attention(const gsvk_t2s_decode_desc* d, size_t l, size_t n, void* x, void* z, void* attn,
+                     const float* qkv, const int64_t* kv_pos, size_t cache_off, const void* ws,
+                     size_t ws_bytes, gsvk::T2sAttnArgs* out) {
+  const size_t D = d->d_model;
+  const gsvk_t2s_layer& L = d->layer[l];
+  gsvk::T2sAttnArgs a{};
+  *out = a;
+  if (d->dtype != GSVK_F16 || d->kv_dtype != GSVK_F16 || d->batch >= kSplitRows ||
+      d->batch * (d->len_bound ? d->len_bound : d->max_len) > kFusedKeys)
+    return false;
+  a.z = l ? z : x, a.x = l ? x : nullptr;
+  a.ln_g = l ? d->layer[l - 1].n2g : nullptr, a.ln_b = l ? d->layer[l - 1].n2b : nullptr;
+  a.wqkv = L.wqkv, a.bqkv = L.bqkv;
+  a.kc = advance(L.k_cache, cache_off), a.vc = advance(L.v_cache, cache_off);
+  a.pos = kv_pos, a.out = attn, a.err = d->err;
+  a.max_len = static_cast<long>(d->max_len), a.heads = static_cast<int>(d->heads);
+  a.eps = static_cast<float>(d->eps), a.inv_n = 1.0 / static_cast<double>(D);
+  a.scale = 1.0f / std::sqrt(static_cast<float>(D / d->heads));
+  if (!gsvk::t2s_qkv_attention_ok(a, n, D)) return false;
+  // scratch the separate launches would write: what they refuse of it stays refused by them
+  const size_t qb = n * 3 * D * sizeof(float), rb = n * D * 2, cb = n * d->max_len * D * 2;
+  if (reinterpret_cast<uintptr_t>(qkv) % 16) return false;
+  const struct { const void* p; size_t n; } other[] = {
+      {a.z, rb}, {a.x, rb}, {a.out, rb}, {a.kc, cb}, {a.vc, cb}};
+  for (const auto& r : other)
+    if (overlap(qkv, qb, r.p, r.n) || overlap(ws, ws_bytes, r.p, r.n)) return false;
+  *out = a;
+  return true;
+}
+
 // One decode step for the rows [b0, b0 + n) of the batch, launch by launch, in block_decode_impl's
 // order. Every launch is row-local (each GEMV row, each sequence's attention and cache rows), so a
 // part of the batch runs exactly as the whole would for those rows; ws is the part's slice of the
@@ -98,7 +154,10 @@ int issue_rows(const gsvk_t2s_decode_desc* d, size_t b0, size_t n, void* ws, siz
   // W1, norm2 into the next layer's QKV or, after the last layer, the logits.
   for (size_t l = 0; l < d->layers; ++l) {
     const gsvk_t2s_layer& L = d->layer[l];
-    if (l == 0) {
+    gsvk::T2sAttnArgs qa;
+    if (fused_attention(d, l, n, x, z, attn, qkv, kv_pos, cache_off, ws, ws_bytes, &qa)) {
+      if ((rc = gsvk::t2s_qkv_attention(qa, n, D, l > 0, st))) return rc;
+    } else if (l == 0) {
       rc = gsvk_gemv_f16w(dt, 1, x, D, L.wqkv, L.bqkv, GSVK_ACT_NONE, 0.f, nullptr, GSVK_F32,
                           qkv, 3 * D, B, 3 * D, D, st);
     } else {  // x = norm2_{l-1}(z), qkv = W_qkv x + b  (t2s_engine.cpp:1119, 1044-1049)
@@ -107,8 +166,8 @@ int issue_rows(const gsvk_t2s_decode_desc* d, size_t b0, size_t n, void* ws, siz
                              GSVK_ACT_NONE, 0.f, nullptr, GSVK_F32, qkv, 3 * D, B, 3 * D, D, st);
     }
     if (rc) return rc;
-    if ((rc = gsvk_decode_attention(d->kv_dtype, dt, qkv, 3 * D,
-                                    advance(L.k_cache, cache_off),
+    if (!qa.z &&
+        (rc = gsvk_decode_attention(d->kv_dtype, dt, qkv, 3 * D, advance(L.k_cache, cache_off),
                                     advance(L.v_cache, cache_off), d->max_len, kv_pos, attn, D,
                                     B, H, D / H, d->len_bound, ws, ws_bytes, d->err, st)))
       return rc;
@@ -130,16 +189,6 @@ int issue_rows(const gsvk_t2s_decode_desc* d, size_t b0, size_t n, void* ws, siz
                              D, st);
   return gsvk_add_layernorm(dt, z, nullptr, nullptr, last.n2g, last.n2b, x, B, D, D, d->eps, st);
 }
-
-// The batch in two parts. At decode sizes every launch but the attention scan is bound by latency,
-// not bandwidth, so the two parts' launch chains are recorded on two streams of one graph, which
-// the runtime issues on two hardware queues and runs side by side. Measured on the whole step
-// (B = 64, 24 layers): 1098 -> 1082-1092 us at 1024 cached keys and 1548-1555 -> 1457-1461 us at
-// 2048. The gain is small because one part's chain alone takes 916-1049 us: the chain's launch
-// latency, not its rows, sets the step time. Batches of fewer than kSplitRows sequences, and
-// workspaces too small for both parts' attention states, run as one part.
-constexpr size_t kSplitRows = 32;
-constexpr size_t kWsAlign = 256;
 
 size_t attn_ws(const gsvk_t2s_decode_desc* d, size_t n) {
   return gsvk_decode_attention_workspace_bytes(n, d->heads, d->d_model / d->heads,
