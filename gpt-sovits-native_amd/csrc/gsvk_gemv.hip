@@ -771,6 +771,225 @@ __global__ __launch_bounds__(kWave * WK) void gemv_stream(GvArgs a) {
   }
 }
 
+// ---- few rows ------------------------------------------------------------------------------------
+//
+// One to four sequences: a launch moves its weights once (0.5 - 2 MB over 256 CUs) and is all
+// latency, and a 16-row matrix-core tile is mostly padding. Here a wave computes R output columns
+// for all rows by itself, in fp32 FMAs on the fp16 operands: each weight row is read as contiguous
+// 1 KiB (lane l holds k = 512 c + 8 l .. + 7), x sits in registers, and the lanes' sums meet by DPP.
+// No LDS and no barrier: with LN every wave forms its own statistics from the row it holds.
+template <int XM>
+struct RowX {  // 8 consecutive k
+  h8 h;        // fp16 x, or fp32 x rounded to fp16
+  __device__ __forceinline__ float get(int i) const { return static_cast<float>(h[i]); }
+};
+template <>
+struct RowX<kXSplit> {
+  f4v a, b;    // fp32 x as it is
+  __device__ __forceinline__ float get(int i) const { return i < 4 ? a[i & 3] : b[i & 3]; }
+};
+
+template <int XM>
+__device__ __forceinline__ RowX<XM> row_x(const float (&v)[8]) {
+  RowX<XM> r;
+  if constexpr (XM == kXSplit) {
+    r.a = f4v{v[0], v[1], v[2], v[3]}, r.b = f4v{v[4], v[5], v[6], v[7]};
+  } else {
+    const u32x4 q = {f2h2(v[0], v[1]), f2h2(v[2], v[3]), f2h2(v[4], v[5]), f2h2(v[6], v[7])};
+    r.h = __builtin_bit_cast(h8, q);
+  }
+  return r;
+}
+
+constexpr int kRowWaves = 4;
+
+template <int XM, bool Y32, int M, int KC, int R, bool LN>
+__global__ __launch_bounds__(kWave * kRowWaves) void gemv_rows(GvArgs a, int ydt) {
+  constexpr int XW = XM == kXF16 ? 1 : 2;  // 16-byte words of x per 8 k
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const long n0 = (static_cast<long>(blockIdx.x) * kRowWaves + wave) * R;
+  if (n0 >= a.N) return;
+  const int K = static_cast<int>(a.K), rows = static_cast<int>(a.M);
+
+  int kc[KC];
+  bool ok[KC];
+#pragma unroll
+  for (int c = 0; c < KC; ++c) {
+    const int k = 512 * c + 8 * lane;
+    ok[c] = k < K;
+    kc[c] = ok[c] ? k : K - 8;
+  }
+  u32x4 xr[M][KC][XW], w[R][KC];
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      const size_t at = static_cast<size_t>(min(m, rows - 1)) * a.ldx + kc[c];
+#pragma unroll
+      for (int q = 0; q < XW; ++q)
+        xr[m][c][q] = XW == 1 ? ld16<false>(static_cast<const uint16_t*>(a.x) + at)
+                              : ld16<false>(static_cast<const float*>(a.x) + at + 4 * q);
+    }
+  u32x4 g[LN ? KC : 1][2], bt[LN ? KC : 1][2];
+  if constexpr (LN) {
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        g[c][q] = ld16<false>(param_or(a.ln_g, kc[c] + 4 * q, kOnes8));
+        bt[c][q] = ld16<false>(param_or(a.ln_b, kc[c] + 4 * q, kZeros8));
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+      w[r][c] = ld16<false>(a.w + static_cast<size_t>(min(n0 + r, a.N - 1)) * a.K + kc[c]);
+  // lane j < R M finishes output (row j / R, column n0 + j % R)
+  const int em = min(lane / R, rows - 1);
+  const long en = min(n0 + lane % R, a.N - 1);
+  const size_t eoff = static_cast<size_t>(em) * a.ldy + en;
+  const float eb = a.bias ? a.bias[en] : 0.f;
+  uint32_t eraw = 0;
+  if (a.res) {
+    if constexpr (Y32) eraw = static_cast<const uint32_t*>(a.res)[eoff];
+    else eraw = static_cast<const uint16_t*>(a.res)[eoff];
+  }
+
+  RowX<XM> x[M][KC];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    float v[KC][8];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      if constexpr (XM == kXF16) {
+        Store<GSVK_F16>::unpack(xr[m][c][0], v[c]);
+      } else {
+        float lo[4], hi[4];
+        Store<GSVK_F32>::unpack(xr[m][c][0], lo);
+        Store<GSVK_F32>::unpack(xr[m][c][XW - 1], hi);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[c][k] = lo[k], v[c][4 + k] = hi[k];
+      }
+    }
+    if constexpr (LN) {  // ln_rows_tile's formulas (csrc/gsvk_norm.hip) in another summation order
+      float s = 0.f;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) s += ok[c] ? chunk_sum<8>(v[c]) : 0.f;
+      const float mean = static_cast<float>(static_cast<double>(wave_sum(s)) * a.inv_n);
+      float q = 0.f;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) q += ok[c] ? chunk_sumsq<8>(v[c], mean) : 0.f;
+      const float var = static_cast<float>(static_cast<double>(wave_sum(q)) * a.inv_n);
+      const float rstd = __builtin_amdgcn_rsqf(var + a.ln_eps);
+      const bool store = a.ln_y && n0 == 0 && m < rows;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const f4v gq = __builtin_bit_cast(f4v, g[c][k / 4]), bq = __builtin_bit_cast(f4v, bt[c][k / 4]);
+          v[c][k] = __builtin_fmaf((v[c][k] - mean) * rstd, gq[k & 3], bq[k & 3]);
+        }
+        const size_t at = static_cast<size_t>(m) * a.ldh + kc[c];
+        if constexpr (XM == kXF16) {
+          const u32x4 hq = Store<GSVK_F16>::pack(v[c]);
+          if (store && ok[c]) st16<false>(static_cast<uint16_t*>(a.ln_y) + at, hq);
+          Store<GSVK_F16>::unpack(hq, v[c]);  // the products see h as it is stored
+        } else if (store && ok[c]) {
+          const float lo[4] = {v[c][0], v[c][1], v[c][2], v[c][3]};
+          const float hi[4] = {v[c][4], v[c][5], v[c][6], v[c][7]};
+          Store<GSVK_F32>::store<false>(a.ln_y, at, lo);
+          Store<GSVK_F32>::store<false>(a.ln_y, at + 4, hi);
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      if (!ok[c]) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[c][k] = 0.f;
+      }
+      x[m][c] = row_x<XM>(v[c]);
+    }
+  }
+
+  float out[R * M];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      float part[KC];
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const h8 wv = __builtin_bit_cast(h8, ok[c] ? w[r][c] : zero);
+        part[c] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          part[c] = __builtin_fmaf(static_cast<float>(wv[k]), x[m][c].get(k), part[c]);
+      }
+      float s = part[0];
+#pragma unroll
+      for (int c = 1; c < KC; ++c) s += part[c];
+      out[m * R + r] = s;
+    }
+  }
+  float v = 0.f;
+  if constexpr (R * M == 1) {
+    v = wave_sum(out[0]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < R * M; j += 2) {
+      float p, q;
+      wave_sum2(out[j], out[j + 1], p, q);
+      v = lane == j ? p : lane == j + 1 ? q : v;
+    }
+  }
+  if (lane >= R * M || lane / R >= rows || n0 + lane % R >= a.N) return;
+  float er = 0.f;
+  if constexpr (Y32) er = __builtin_bit_cast(float, eraw);
+  else er = ydt == GSVK_F16 ? h2f(eraw) : bf2f(eraw);
+  v = epilogue(a, v, eb, er);
+  if constexpr (Y32) static_cast<float*>(a.y)[eoff] = v;
+  else static_cast<uint16_t*>(a.y)[eoff] = static_cast<uint16_t>(ydt == GSVK_F16 ? f2h(v) : f2bf(v));
+}
+
+// Up to 4 rows of up to 2048 inputs (the shapes it is laid out for; a wave must hold x), and not the
+// long streams, whose kernel reads the weights better.
+#ifndef ROWS_MAX
+#define ROWS_MAX 4
+#endif
+bool few_rows(long M, long N, long K) { return M <= ROWS_MAX && K >= 256 && K <= 2048 && N <= 16384; }
+
+template <int XM, bool Y32, int M, int KC, int R, bool LN>
+void launch_rows_r(const GvArgs& a, int ydt, hipStream_t st) {
+  const long blocks = (a.N + kRowWaves * R - 1) / (kRowWaves * R);
+  hipLaunchKernelGGL((gemv_rows<XM, Y32, M, KC, R, LN>), dim3(static_cast<unsigned>(blocks)),
+                     dim3(kWave * kRowWaves), 0, st, a, ydt);
+}
+
+// Two columns per wave from 1024 columns on (512 waves: two per CU); below, one.
+template <int XM, bool Y32, int M, int KC, bool LN>
+void launch_rows_kc(const GvArgs& a, int ydt, hipStream_t st) {
+  if (a.N >= 1024) return launch_rows_r<XM, Y32, M, KC, 2, LN>(a, ydt, st);
+  return launch_rows_r<XM, Y32, M, KC, 1, LN>(a, ydt, st);
+}
+
+template <int XM, bool Y32, int M, bool LN>
+void launch_rows_m(const GvArgs& a, int ydt, hipStream_t st) {
+  if (a.K <= 512) return launch_rows_kc<XM, Y32, M, 1, LN>(a, ydt, st);
+  if (LN || a.K <= 1024) return launch_rows_kc<XM, Y32, M, 2, LN>(a, ydt, st);
+  if constexpr (!LN) launch_rows_kc<XM, Y32, M, 4, LN>(a, ydt, st);
+}
+
+template <int XM, int YDT, bool LN>
+void launch_rows(const GvArgs& a, hipStream_t st) {
+  constexpr bool Y32 = YDT == GSVK_F32;
+  if (a.M == 1) return launch_rows_m<XM, Y32, 1, LN>(a, YDT, st);
+  return launch_rows_m<XM, Y32, 4, LN>(a, YDT, st);
+}
+
 // ---- launch plan ---------------------------------------------------------------------------------
 
 template <int XM, int YDT, int MF, int NF, int WK, int D, bool LN>
@@ -849,6 +1068,7 @@ void launch_stream(const GvArgs& a, hipStream_t st) {
 
 template <int XM, int YDT, bool LN>
 void launch_plan(const GvArgs& a, bool tiled, hipStream_t st) {
+  if (tiled && few_rows(a.M, a.N, a.K)) return launch_rows<XM, YDT, LN>(a, st);
   if constexpr (!LN) {
     const long tiles = (a.N + 15) / 16 * ((a.M + 15) / 16);
     if (stream_ok(a, tiled, tiles, YDT == GSVK_F32 ? 4 : 2, XM == kXSplit))
