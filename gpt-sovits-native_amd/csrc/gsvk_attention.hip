@@ -308,6 +308,156 @@ __global__ __launch_bounds__(kWave * kMaxChunks) void attn_merge(AttnArgs a, int
   store8<OUTT>(a.out, static_cast<size_t>(b) * a.ldo + 8 * lane, y);
 }
 
+// ---- heads split over workgroups -----------------------------------------------------------------
+//
+// With enough sequences the work is split by heads instead of by keys: a workgroup scans all keys of
+// one sequence for the heads in LPK lanes x 8 dims (a 16 LPK-byte piece of each 16-bit row), so every
+// softmax is finished where it was begun. No chunk states, no second launch. 64 / LPK keys per
+// load instruction, kSlots instructions of K and of V in flight per wave; the scores of kSlots x
+// 64 / LPK keys share one rescaling of the running state.
+constexpr int kHeadSlots = 4;
+constexpr int kHeadWaves = 8;
+
+template <int KVT, int OUTT, int LPK, bool NT>
+__global__ __launch_bounds__(kWave * kHeadWaves) void attn_heads(AttnArgs a) {
+  constexpr int KPW = kWave / LPK;  // keys per wave and instruction
+  constexpr int KPR = KPW * kHeadWaves;
+  constexpr int W = KeyGroup<KVT>::W;
+  constexpr size_t kEsz = KVT == GSVK_F32 ? 4 : 2;
+  __shared__ float st_m[kHeadWaves][LPK], st_l[kHeadWaves][LPK], st_o[kHeadWaves][8][LPK];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int sub = lane / LPK, dl = lane % LPK;
+  const long b = blockIdx.y, D = a.D;
+  const int lpd = static_cast<int>(a.HD / 8);
+  const size_t col = static_cast<size_t>(blockIdx.x) * (LPK * 8) + 8 * dl;
+
+  const int64_t pos = a.pos[b];
+  const bool valid = pos >= 0 && pos < a.max_len;
+  const int past = valid ? static_cast<int>(pos) : 0;  // cached keys before the new one
+  const int rounds = (past + KPR - 1) / KPR;
+  const size_t seq = static_cast<size_t>(b) * a.max_len * D + col;
+  const int key0 = wave * KPW + sub;
+  u32x4 kr[kHeadSlots][W], vr[kHeadSlots][W];
+  auto at = [&](int r) {  // past the end: the last cached key again, with weight 0
+    return (seq + static_cast<size_t>(max(0, min(key0 + KPR * r, past - 1))) * D) * kEsz;
+  };
+  auto k_load = [&](int s, int r) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) kr[s][w] = ld16<NT>(static_cast<const char*>(a.kc) + at(r) + 16 * w);
+  };
+  auto v_load = [&](int s, int r) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) vr[s][w] = ld16<NT>(static_cast<const char*>(a.vc) + at(r) + 16 * w);
+  };
+#pragma unroll
+  for (int s = 0; s < kHeadSlots; ++s) k_load(s, s);
+#pragma unroll
+  for (int s = 0; s < kHeadSlots; ++s) v_load(s, s);
+
+  const float* qrow = a.qkv + b * a.ldq + col;
+  float q[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) q[i] = qrow[i];
+  // Maxima start at the lowest finite value: differences below are numbers or -inf (weight 0).
+  float m = -3.4028234663852886e38f, l = 0.f, o[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = 0.f;
+  if (wave == 0) {  // the new token: the first LPK lanes of wave 0; the append
+    float kn[8], vn[8], d = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      kn[i] = round_to<KVT>(qrow[D + i]);
+      vn[i] = round_to<KVT>(qrow[2 * D + i]);
+      d = __builtin_fmaf(q[i], kn[i], d);
+    }
+    d = head_sum(d, lpd) * a.scale;
+    if (sub == 0 && valid) {
+      m = fmaxf(m, d);
+      l = __expf(d - m);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = l * vn[i];
+      store8<KVT>(a.kc, seq + static_cast<size_t>(pos) * D, kn);
+      store8<KVT>(a.vc, seq + static_cast<size_t>(pos) * D, vn);
+    }
+  }
+  for (int r0 = 0; r0 < rounds; r0 += kHeadSlots) {
+    float sc[kHeadSlots], mn = m;
+#pragma unroll
+    for (int s = 0; s < kHeadSlots; ++s) {
+      float kf[8], d = 0.f;
+      unpack8<KVT>(kr[s], kf);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) d = __builtin_fmaf(q[i], kf[i], d);
+      d = head_sum(d, lpd) * a.scale;
+      sc[s] = key0 + KPR * (r0 + s) < past ? d : -INFINITY;
+      mn = fmaxf(mn, sc[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < kHeadSlots; ++s) k_load(s, r0 + kHeadSlots + s);
+    const float corr = __expf(m - mn);
+    m = mn;
+    l *= corr;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] *= corr;
+#pragma unroll
+    for (int s = 0; s < kHeadSlots; ++s) {
+      float vf[8];
+      unpack8<KVT>(vr[s], vf);
+      const float p = __expf(sc[s] - mn);
+      l += p;
+      if (key0 + KPR * (r0 + s) < past) {  // (0 times an infinite value of the reread row is NaN)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = __builtin_fmaf(p, vf[i], o[i]);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < kHeadSlots; ++s) v_load(s, r0 + kHeadSlots + s);
+  }
+
+  // the wave's 64 / LPK key lanes, then the waves in order
+  float M = m;
+#pragma unroll
+  for (int off = LPK; off < kWave; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, kWave));
+  const float f = __expf(m - M);
+  l *= f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] *= f;
+#pragma unroll
+  for (int off = LPK; off < kWave; off <<= 1) {
+    l += __shfl_xor(l, off, kWave);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] += __shfl_xor(o[i], off, kWave);
+  }
+  if (sub == 0) {
+    st_m[wave][dl] = M;
+    st_l[wave][dl] = l;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) st_o[wave][i][dl] = o[i];
+  }
+  __syncthreads();
+  if (wave != 0 || sub != 0) return;
+  M = st_m[0][dl];
+#pragma unroll
+  for (int w = 1; w < kHeadWaves; ++w) M = fmaxf(M, st_m[w][dl]);
+  float L = 0.f, O[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) O[i] = 0.f;
+#pragma unroll
+  for (int w = 0; w < kHeadWaves; ++w) {
+    const float e = __expf(st_m[w][dl] - M);
+    L = __builtin_fmaf(st_l[w][dl], e, L);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) O[i] = __builtin_fmaf(st_o[w][i][dl], e, O[i]);
+  }
+  float y[8];
+  const float inv = 1.f / L;  // L = 0 only for an invalid position: NaN row
+#pragma unroll
+  for (int i = 0; i < 8; ++i) y[i] = L > 0.f ? O[i] * inv : __builtin_nanf("");
+  store8<OUTT>(a.out, static_cast<size_t>(b) * a.ldo + col, y);
+  if (!valid && blockIdx.x == 0 && lane == 0 && a.err) *a.err = 1;
+}
+
 // Key chunks per sequence: one round of at most one workgroup per CU, 4 chunks at B = 64 on 256
 // CUs. The workgroups of a launch stream their keys in step, so a partly filled last round costs a
 // whole one. Measured on the whole T2S decode step (B = 64, 1024 and 2048 cached keys, non-temporal
@@ -326,8 +476,48 @@ int chunks_for(size_t batch, size_t len_bound) {
   return static_cast<int>(std::max(1L, std::min<long>(c, kMaxChunks)));
 }
 
+// Lanes per key of attn_heads for this call, 0: the key chunks. A workgroup's piece of a row holds
+// whole heads and divides D; of those, the narrowest that still runs all workgroups in one round of
+// one per CU (64-byte pieces, half a cache line, were slower throughout). With 16-bit caches the split
+// by heads wins from 24 sequences on, and below that up to about 1000 keys, past which the chunks'
+// finer split of the few sequences pays for their merge; with fp32 rows (twice the bytes per piece)
+// from 48, and up to 500 keys. Per call, chunks + merge against heads, cold caches, contexts ragged
+// over a third of the given: 64 x 1024 26.4 -> 22.1 us, 64 x 2048 45.5 -> 38.1, 64 x 100 10.1 -> 5.8,
+// 128 x 1024 45.2 -> 37.6, 24 x 1500 18.7 -> 17.4, 16 x 300 10.3 -> 6.3, 8 x 500 10.3 -> 6.2;
+// 8 x 1500 13.1 -> 14.7, 20 x 2000 19.9 -> 20.8; fp32 64 x 1024 50.0 -> 46.9, 24 x 1500 33.2 -> 39.2.
+int head_lanes(const AttnArgs& a, size_t B, size_t esz, size_t len_bound) {
+  const bool f32 = esz == 4;
+  if (B < (f32 ? 48 : 24) && len_bound * esz > 2000) return 0;
+  const long lanes = a.D / 8, lpd = a.HD / 8;
+  int best = 0;
+  for (int lpk = 64; lpk >= 8; lpk /= 2) {
+    if (lpk % lpd || lanes % lpk) continue;
+    if (best && static_cast<long>(B) * (lanes / lpk) > device_cus()) break;
+    best = lpk;
+  }
+  // 128-byte pieces of long contexts lose to whole rows again when another call shares the HBM: the
+  // halves of a 64 x 2000 decode step 1467 -> 1559 us (alone, 24 x 2000 22.5 -> 21.6).
+  return best == 8 && len_bound * esz > 3400 ? 0 : best;
+}
+
+template <int KVT, int OUTT, int LPK>
+void launch_heads(const AttnArgs& a, size_t B, bool nt, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(a.D / (8 * LPK)), static_cast<unsigned>(B));
+  if (nt)
+    hipLaunchKernelGGL((attn_heads<KVT, OUTT, LPK, true>), grid, dim3(kWave * kHeadWaves), 0, st, a);
+  else
+    hipLaunchKernelGGL((attn_heads<KVT, OUTT, LPK, false>), grid, dim3(kWave * kHeadWaves), 0, st, a);
+}
+
 template <int KVT, int OUTT>
-void launch_attn(const AttnArgs& a, size_t B, int C, bool nt, hipStream_t st) {
+void launch_attn(const AttnArgs& a, size_t B, int C, bool nt, size_t len_bound, hipStream_t st) {
+  switch (head_lanes(a, B, KVT == GSVK_F32 ? 4 : 2, len_bound)) {
+    case 8: return launch_heads<KVT, OUTT, 8>(a, B, nt, st);
+    case 16: return launch_heads<KVT, OUTT, 16>(a, B, nt, st);
+    case 32: return launch_heads<KVT, OUTT, 32>(a, B, nt, st);
+    case 64: return launch_heads<KVT, OUTT, 64>(a, B, nt, st);
+    default: break;
+  }
   const dim3 grid(C, static_cast<unsigned>(B));
   if (nt)
     hipLaunchKernelGGL((attn_chunk<KVT, OUTT, true>), grid, dim3(kWave * kAttnWaves), 0, st, a);
@@ -339,11 +529,11 @@ void launch_attn(const AttnArgs& a, size_t B, int C, bool nt, hipStream_t st) {
 }
 
 template <int KVT>
-void launch_out(int outt, const AttnArgs& a, size_t B, int C, bool nt, hipStream_t st) {
+void launch_out(int outt, const AttnArgs& a, size_t B, int C, bool nt, size_t lb, hipStream_t st) {
   switch (outt) {
-    case GSVK_F32: return launch_attn<KVT, GSVK_F32>(a, B, C, nt, st);
-    case GSVK_F16: return launch_attn<KVT, GSVK_F16>(a, B, C, nt, st);
-    default: return launch_attn<KVT, GSVK_BF16>(a, B, C, nt, st);
+    case GSVK_F32: return launch_attn<KVT, GSVK_F32>(a, B, C, nt, lb, st);
+    case GSVK_F16: return launch_attn<KVT, GSVK_F16>(a, B, C, nt, lb, st);
+    default: return launch_attn<KVT, GSVK_BF16>(a, B, C, nt, lb, st);
   }
 }
 
@@ -415,9 +605,9 @@ __attribute__((visibility("hidden"))) int attention_call(
   const size_t keys = len_bound ? std::min(len_bound, max_len) : max_len;
   const bool nt = 2 * batch * keys * D * esz >= kAttnStreamBytes;
   switch (kv_dtype) {
-    case GSVK_F32: launch_out<GSVK_F32>(out_dtype, a, batch, C, nt, st); break;
-    case GSVK_F16: launch_out<GSVK_F16>(out_dtype, a, batch, C, nt, st); break;
-    default: launch_out<GSVK_BF16>(out_dtype, a, batch, C, nt, st); break;
+    case GSVK_F32: launch_out<GSVK_F32>(out_dtype, a, batch, C, nt, keys, st); break;
+    case GSVK_F16: launch_out<GSVK_F16>(out_dtype, a, batch, C, nt, keys, st); break;
+    default: launch_out<GSVK_BF16>(out_dtype, a, batch, C, nt, keys, st); break;
   }
   return launch_status();
 }

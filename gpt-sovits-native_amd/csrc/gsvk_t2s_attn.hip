@@ -211,8 +211,10 @@ __attribute__((amdgpu_waves_per_eu(2))) void t2s_qkv_attn(T2sAttnArgs a) {
     for (int s = 0; s < kSlots; ++s) {
       const float p = __expf(sc[s] - mn);
       l += p;
+      if (key0 + kKeysPerRound * (r0 + s) < past) {  // (0 times an infinite reread value is NaN)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = __builtin_fmaf(p, static_cast<float>(vr[s][i]), o[i]);
+        for (int i = 0; i < 8; ++i) o[i] = __builtin_fmaf(p, static_cast<float>(vr[s][i]), o[i]);
+      }
     }
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) v_load(s, r0 + kSlots + s);

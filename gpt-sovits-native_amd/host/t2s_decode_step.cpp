@@ -71,14 +71,16 @@ T* advance(T* p, size_t bytes) {
   return p ? reinterpret_cast<T*>(reinterpret_cast<B*>(p) + bytes) : nullptr;
 }
 
-// The batch in two parts. At decode sizes every launch but the attention scan is bound by latency,
-// not bandwidth, so the two parts' launch chains are recorded on two streams of one graph, which
-// the runtime issues on two hardware queues and runs side by side. Measured on the whole step
-// (B = 64, 24 layers): 1098 -> 1082-1092 us at 1024 cached keys and 1548-1555 -> 1457-1461 us at
-// 2048. The gain is small because one part's chain alone takes 916-1049 us: the chain's launch
-// latency, not its rows, sets the step time. Batches of fewer than kSplitRows sequences, and
-// workspaces too small for both parts' attention states, run as one part.
+// The batch in two parts, for long contexts: the two parts' launch chains are recorded on two streams
+// of one graph, which the runtime issues on two hardware queues, so one part's latency-bound GEMVs
+// overlap the other's key scan. Every launch of a part costs nearly what it costs for the whole
+// batch, so the scan has to be long for that to pay. Whole step (24 layers), us, one chain against two
+// halves: 64 x 300 714 / 792, 64 x 1024 1001 / 1037, 64 x 1500 1213 / 1260, 64 x 2000 1555 / 1467,
+// 32 x 2000 1029 / 1095, 128 x 600 1212 / 1220 (the halves' better time of either attention form).
+// Batches of fewer than kSplitRows sequences, and workspaces too small for both parts' attention
+// states, run as one part too.
 constexpr size_t kSplitRows = 32;
+constexpr size_t kSplitKeys = 110000;  // batch x len_bound
 constexpr size_t kWsAlign = 256;
 
 // The fused launch reads W_qkv once per sequence and its keys in 64-byte pieces: it wins while few
@@ -201,9 +203,15 @@ struct Part {
   size_t ws_bytes;
 };
 
-int parts_of(const gsvk_t2s_decode_desc* d, Part (&p)[2]) {
+size_t keys_bound(const gsvk_t2s_decode_desc* d) {
+  return d->len_bound ? d->len_bound : d->max_len;
+}
+
+// any_length: the parts of long contexts, whatever the descriptor's.
+int parts_of(const gsvk_t2s_decode_desc* d, Part (&p)[2], bool any_length = false) {
   const size_t B = d->batch;
-  if (d->parts != 1 && B >= kSplitRows && d->workspace) {
+  if (d->parts != 1 && B >= kSplitRows && d->workspace &&
+      (any_length || B * keys_bound(d) > kSplitKeys)) {
     const size_t n0 = B / 2, n1 = B - n0;
     const size_t w0 = (attn_ws(d, n0) + kWsAlign - 1) / kWsAlign * kWsAlign, w1 = attn_ws(d, n1);
     if (d->workspace_bytes >= w0 + w1) {
@@ -236,9 +244,11 @@ int count_part_launches(const gsvk_t2s_decode_desc* d, const Part& p) {
   return static_cast<int>(1 + d->layers * (merge ? 6 : 5) + 1);
 }
 
+// The passes of a step: those of the two halves where parts 0 allows them, of the separate launches
+// of each layer, whichever form runs.
 int count_decode_launches(const gsvk_t2s_decode_desc* d) {
   Part p[2];
-  const int np = parts_of(d, p);
+  const int np = parts_of(d, p, true);
   int n = 0;
   for (int i = 0; i < np; ++i) n += count_part_launches(d, p[i]);
   return n;

@@ -173,7 +173,8 @@ int gsvk_gemv_f16w_ln(int x_dtype, int round_x, const void* z, size_t ldz, const
  * whatever its value (the partition of the keys, so the rounding, follows it). With more
  * than one chunk the partial states go through `workspace` (gsvk_decode_attention_workspace_bytes
  * bytes, 16-byte aligned; no initialisation needed); with a NULL or smaller workspace every sequence
- * runs as one chunk. Cache rows at and past pos[b] may hold any bits (stale, Inf, NaN): none of
+ * runs as one chunk. (With enough sequences, or few keys, the work is split by heads instead, and the
+ * workspace is not written.) Cache rows at and past pos[b] may hold any bits (stale, Inf, NaN): none of
  * them enters the result. A position outside [0, max_len) (undefined in the reference) writes a
  * NaN row, leaves the caches untouched and stores 1 into *err when err != NULL.
  * The softmax is formed online (running maximum, rescaled sums) in another order than the

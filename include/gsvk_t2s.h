@@ -160,10 +160,11 @@ typedef struct gsvk_t2s_decode_desc {
   float* qkv;/* [B, 3D] */
   void* workspace;         /* gsvk_t2s_decode_workspace_bytes(batch, heads, D/heads, len)     */
   size_t workspace_bytes;
-  int parts;               /* 0: two halves when batch >= 32, else one chain; 1: one chain    */
+  int parts;               /* 0: two halves for large batches of long contexts; 1: one chain   */
 } gsvk_t2s_decode_desc;
 
-/* With parts 0 a batch of 32 sequences or more runs as two halves, when the workspace holds both
+/* With parts 0 a batch of 32 sequences or more over long contexts (batch x len_bound above 110000)
+ * runs as two halves, when the workspace holds both
  * halves' attention states (gsvk_t2s_decode_workspace_bytes; otherwise as one chain): every launch
  * is row-local, so each half is the same chain of launches over its rows, and the graph records the
  * two chains on two branches that run concurrently (one half's latency-bound GEMVs overlap the
