@@ -116,17 +116,29 @@ def lib():
 
 def _ptr(t):
     """Device address of a torch tensor (or an int address / None)."""
-    if t is None:
-        return None
-    if isinstance(t, int):
+    if t is None or isinstance(t, int):
         return t
     return t.data_ptr()
 
 
+_RAW_STREAM = []
+
+
+def _current_stream():
+    """Handle of torch's current stream on the current device. torch.cuda.current_stream() builds a
+    Stream object behind three device lookups (3 us a call, a third of what a short launch costs
+    from Python); torch's own launchers read the handle this way."""
+    if not _RAW_STREAM:
+        import torch
+        torch.cuda.current_stream()  # initialises CUDA, or raises as it does
+        _RAW_STREAM[:] = (torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice)
+    raw, device = _RAW_STREAM
+    return raw(device())
+
+
 def _stream(stream):
     if stream is None:
-        import torch
-        return torch.cuda.current_stream().cuda_stream
+        return _current_stream()
     return stream if isinstance(stream, int) else stream.cuda_stream
 
 
@@ -154,11 +166,14 @@ def dtype_code(t):
 
 def _rows(t):
     """(rows, n, ld) of a 2-D row-major view (or a 1-D buffer as one row)."""
-    if t.dim() == 1:
-        return 1, t.shape[0], t.shape[0]
-    assert t.dim() == 2 and (t.stride(1) == 1 or t.shape[1] == 1), "rows must be contiguous"
+    shape = t.shape
+    if len(shape) == 1:
+        return 1, shape[0], shape[0]
+    assert len(shape) == 2, "rows must be contiguous"
+    (rows, n), (ld, step) = shape, t.stride()
+    assert step == 1 or n == 1, "rows must be contiguous"
     # a single row has no meaningful row stride (numpy / torch may report 0 for it)
-    return t.shape[0], t.shape[1], t.stride(0) if t.shape[0] > 1 else t.shape[1]
+    return rows, n, ld if rows > 1 else n
 
 
 def add_layernorm(x, gamma, beta, y, eps, bias=None, residual=None, stream=None, check=True):
