@@ -948,6 +948,265 @@ int launch_ks(const ConvArgs* a, int n, hipStream_t st) {
   return launch_ksplit<XM, 4, 2, 4, 2, 4>(a, n, st);
 }
 
+// ---- a ResBlock pair of a narrow stage in one launch ------------------------------------------------
+//
+// out = x + (W2 * lrelu(W1 *_dil lrelu(x) + b1) + b2) for up to 96 channels, where one workgroup holds
+// every channel of its columns. The two convolutions of such a pair are bound by their short load ->
+// stage -> multiply -> store sequences and by the activations' traffic (x read, t_a written and read,
+// x read again, the sum written), not by their products. Here t_a never leaves LDS: a workgroup
+// computes kPairCols columns of t_a (its outputs' and the k - 1 the second convolution reaches past
+// them), writes them over the staged x in the staging layout and multiplies again. Waves side by side
+// along t as in conv1d_mfma; the weights go straight from L1 / L2 into the fragments, D units ahead
+// across both convolutions (all four waves read the same), so the only barriers are around the two
+// changes of LDS contents. Sums in conv1d_mfma's order: the same bits as the two launches.
+//
+// Measured on the whole decoder (graph), the 48- and 24-channel stages' pairs as two launches against
+// one: 75 frames fp16 670 -> 598 us, 500 frames fp16 1923 -> 1791, exact fp32 2719 -> 2595; the
+// 96-channel stage too: 75 frames 600 -> 582, 500 frames exact -> 2574 (40 frames 469 -> 488: not
+// below 8192 columns). Two units ahead and four waves per SIMD up to 48 channels; four or six units
+// ahead at three waves were 2-5% slower on the fp16 decoder.
+struct PairArgs {
+  ConvArgs a1, a2;  // a1: x, lrelu in and out; a2: the residual sum into cur
+  int tth;          // staged columns of x: kPairCols + halo, a multiple of 16
+  uint32_t tth_inv;
+  int out_cols;     // outputs per workgroup
+  int esz_row;
+};
+constexpr int kPairCols = kWaves * 32;
+constexpr int kPairTa = kPairCols + 16;  // columns of t_a in LDS: the taps of the last outputs
+
+template <int XM, int NO, int D>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(NO > 3 ? 2 : 4))) void conv_pair(PairArgs p) {
+  constexpr int DT = storage_dt<XM>();
+  constexpr int P = planes<XM>();
+  constexpr int NT = 2;
+  constexpr int ESZ = DT == GSVK_F32 ? 4 : 2;
+  extern __shared__ __attribute__((aligned(16))) _Float16 xs[];
+  const ConvArgs& a = p.a1;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r16 = lane & 15, grp = lane >> 4;
+  const long tile = a.xspan ? static_cast<long>(blockIdx.x % kXcds) * a.xspan + blockIdx.x / kXcds
+                            : static_cast<long>(blockIdx.x);
+  const long t0 = tile * p.out_cols;
+  if (t0 >= a.T) return;
+  const int T = static_cast<int>(a.T), C = static_cast<int>(a.cin), nch = a.nch, k = a.k;
+  const int pad2 = p.a2.pad;
+
+  // ---- weights: unit s = chunk x tap of the first convolution, then of the second ---------------
+  const int nu = nch * k;
+  const int unit_bytes = static_cast<int>(a.opad) * 4 * 16;
+  const __amdgpu_buffer_rsrc_t w1 = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(a.wp), 0, nu * unit_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t w2 = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(p.a2.wp), 0, nu * unit_bytes, 0x00020000);
+  const int wofs = (grp * static_cast<int>(a.opad) + r16) * 16;
+  u32x4 wr[D][NO];
+  auto wload = [&](u32x4 (&w)[NO], const __amdgpu_buffer_rsrc_t rs, int s) {
+#pragma unroll
+    for (int n = 0; n < NO; ++n)
+      w[n] = __builtin_amdgcn_raw_buffer_load_b128(rs, wofs + 16 * 16 * n, s * unit_bytes, 0);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) wload(wr[d], w1, min(d, nu - 1));
+
+  // ---- x: every channel of columns t0 - pad2 - pad .. + tth - 1 -----------------------------------
+  const int tbase = static_cast<int>(t0) - pad2 - a.pad, tth = p.tth;
+  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(a.x), 0, (C - 1) * p.esz_row + T * ESZ, 0x00020000);
+  float m1 = -1.f;
+  asm("" : "+s"(m1));
+  const int items = nch * 4 * tth;
+  constexpr int U = 3;
+  for (int i0 = 0; i0 < items; i0 += kThreads * U) {
+    uint32_t raw[U][8];
+    bool ok[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int it = min(i0 + tid + kThreads * u, items - 1);
+      const int g = static_cast<int>(__umulhi(static_cast<uint32_t>(it), p.tth_inv));  // it / tth
+      const int t = tbase + it - g * tth, ch = 8 * g;
+      ok[u] = t >= 0 && t < T && ch < C;
+      const int off = min(ch, C - 8) * p.esz_row + min(max(t, 0), T - 1) * ESZ;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if constexpr (DT == GSVK_F32)
+          raw[u][j] = __builtin_amdgcn_raw_buffer_load_b32(xrs, off, j * p.esz_row, 0);
+        else
+          raw[u][j] = __builtin_amdgcn_raw_buffer_load_b16(xrs, off, j * p.esz_row, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int it = i0 + tid + kThreads * u;
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j] = DT == GSVK_F32 ? __builtin_bit_cast(float, raw[u][j]) : h2f(raw[u][j]);
+        v[j] = lrelu_ref(ok[u] ? v[j] : 0.f, a.slope);
+      }
+      if (it < items) {
+        if constexpr (P == 2) {
+          const u32x4 hi = {pack_h2(v[0], v[1]), pack_h2(v[2], v[3]), pack_h2(v[4], v[5]),
+                            pack_h2(v[6], v[7])};
+          const u32x4 lo = {split_rest2(hi[0], v[0], v[1], m1), split_rest2(hi[1], v[2], v[3], m1),
+                            split_rest2(hi[2], v[4], v[5], m1), split_rest2(hi[3], v[6], v[7], m1)};
+          *reinterpret_cast<u32x4*>(xs + static_cast<size_t>(it) * 8) = hi;
+          *reinterpret_cast<u32x4*>(xs + static_cast<size_t>(items + it) * 8) = lo;
+        } else {
+          *reinterpret_cast<u32x4*>(xs + static_cast<size_t>(it) * 8) =
+              u32x4{f2h2(v[0], v[1]), f2h2(v[2], v[3]), f2h2(v[4], v[5]), f2h2(v[6], v[7])};
+        }
+      }
+    }
+  }
+  // biases: of the 4 consecutive channels a lane's first results are, of its row in the second's
+  float b1[NO][4], b2[NO];
+#pragma unroll
+  for (int n = 0; n < NO; ++n) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) b1[n][q] = a.bias ? a.bias[min(16 * n + 4 * grp + q, C - 1)] : 0.f;
+    b2[n] = p.a2.bias ? p.a2.bias[min(16 * n + r16, C - 1)] : 0.f;
+  }
+  __syncthreads();
+
+  // ---- the units of one convolution over LDS rows of `cols` columns, tap shift `dil`; SWAP: channels
+  // in the accumulator's registers (D = W X), otherwise positions (D = X W) -------------------------
+  f4v acc[NT][NO];
+  auto conv = [&](auto swap, int cols, int dil, auto next) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int n = 0; n < NO; ++n) acc[i][n] = f4v{0.f, 0.f, 0.f, 0.f};
+    int c = 0, kk = 0;
+    for (int j0 = 0; j0 < nu; j0 += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        if (j0 + d < nu) {
+          const _Float16* xw = xs + (static_cast<size_t>(c * 4 + grp) * cols + wave * 32 + r16 +
+                                     kk * dil) * 8;
+          h8 xf[NT][P];
+#pragma unroll
+          for (int q = 0; q < P; ++q)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+              xf[i][q] = *reinterpret_cast<const h8*>(
+                  xw + (static_cast<size_t>(q) * nch * 4 * cols + 16 * i) * 8);
+#pragma unroll
+          for (int q = 0; q < P; ++q)
+#pragma unroll
+            for (int n = 0; n < NO; ++n)
+#pragma unroll
+              for (int i = 0; i < NT; ++i) {
+                const h8 wv = __builtin_bit_cast(h8, wr[d][n]);
+                if constexpr (decltype(swap)::value)
+                  acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xf[i][q], acc[i][n], 0, 0, 0);
+                else
+                  acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[i][q], wv, acc[i][n], 0, 0, 0);
+              }
+          if (++kk == k) kk = 0, ++c;
+        }
+        next(d, j0 + D + d);
+      }
+    }
+  };
+  // slot d's next unit; past the first convolution, the second's unit d
+  conv(std::true_type{}, tth, a.dil, [&](int d, int u) {
+    if (u < nu) wload(wr[d], w1, u);
+    else wload(wr[d], w2, min(d, nu - 1));
+  });
+  __syncthreads();
+
+  // ---- t_a over x: lane's 4 channels 16 n + 4 grp .. of column wave 32 + 16 i + r16 ----------------
+  const size_t plane = static_cast<size_t>(nch) * 4 * kPairTa * 8;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const int col = wave * 32 + 16 * i + r16;
+    const int t = static_cast<int>(t0) - pad2 + col;
+    const bool in = t >= 0 && t < T;
+#pragma unroll
+    for (int n = 0; n < NO; ++n) {
+      const int o = 16 * n + 4 * grp;
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v[q] = a.bias ? acc[i][n][q] + b1[n][q] : acc[i][n][q];
+        v[q] = in && o + q < C ? lrelu_ref(v[q], a.slope) : 0.f;
+      }
+      _Float16* at = xs + (static_cast<size_t>(o / 8) * kPairTa + col) * 8 + o % 8;
+      if constexpr (P == 2) {
+        const uint2 hi = {pack_h2(v[0], v[1]), pack_h2(v[2], v[3])};
+        *reinterpret_cast<uint2*>(at) = hi;
+        *reinterpret_cast<uint2*>(at + plane) =
+            uint2{split_rest2(hi.x, v[0], v[1], m1), split_rest2(hi.y, v[2], v[3], m1)};
+      } else {
+        *reinterpret_cast<uint2*>(at) = uint2{f2h2(v[0], v[1]), f2h2(v[2], v[3])};
+      }
+    }
+  }
+  // channel groups past the computed rows (their weights are zero, their LDS must be finite)
+  const int pad_rows = (nch * 4 - 2 * NO) * kPairTa;
+  for (int e = tid; e < P * pad_rows; e += kThreads) {
+    const int q = P == 2 && e >= pad_rows ? 1 : 0, r = e - q * pad_rows;
+    *reinterpret_cast<u32x4*>(xs + q * plane + (static_cast<size_t>(2 * NO) * kPairTa + r) * 8) =
+        u32x4{0u, 0u, 0u, 0u};
+  }
+  const Map m = block_map(p.a2, 0);
+  f4v cur[NT][NO];
+#pragma unroll
+  for (int n = 0; n < NO; ++n)
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+      cur[i][n] = load_cur<DT>(p.a2, m, 16 * n + r16, t0 + wave * 32 + 16 * i + 4 * grp);
+  __syncthreads();
+
+  conv(std::false_type{}, kPairTa, 1, [&](int d, int u) { wload(wr[d], w2, min(u, nu - 1)); });
+#pragma unroll
+  for (int n = 0; n < NO; ++n) {
+    const int o = 16 * n + r16;
+    if (o >= C) continue;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int col = wave * 32 + 16 * i + 4 * grp;
+      const long t = t0 + col;
+      if (col < p.out_cols && t < a.T) finish4<DT>(p.a2, m, o, t, acc[i][n], b2[n], cur[i][n]);
+    }
+  }
+}
+
+template <int XM, int NO>
+int launch_pair(const ConvArgs& a1, const ConvArgs& a2, hipStream_t st) {
+  auto kern = conv_pair<XM, NO, 2>;
+  PairArgs p{};
+  p.a1 = a1, p.a2 = a2;
+  p.tth = (kPairCols + a1.halo + 15) / 16 * 16;
+  p.tth_inv = static_cast<uint32_t>(((1ull << 32) + p.tth - 1) / p.tth);
+  p.out_cols = (kPairCols - (a1.k - 1)) / 4 * 4;
+  p.esz_row = static_cast<int>(a1.ldx) * (storage_dt<XM>() == GSVK_F32 ? 4 : 2);
+  const size_t lds = static_cast<size_t>(planes<XM>()) * a1.nch * 4 * std::max(p.tth, kPairTa) * 16;
+  if constexpr (NO > 3) {
+    static std::atomic<bool> lds_ok[kMaxDevices];
+    if (!allow_dynamic_lds(reinterpret_cast<const void*>(kern), 96 * 1024, lds_ok)) return GSVK_E_HIP;
+  }
+  const long gx = (a1.T + p.out_cols - 1) / p.out_cols;
+  p.a1.xspan = gx >= kXcdMinTiles ? (gx + kXcds - 1) / kXcds : 0;
+  const long gxl = p.a1.xspan ? p.a1.xspan * kXcds : gx;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(gxl)), dim3(kThreads), lds, st, p);
+  return launch_status();
+}
+
+template <int XM>
+int launch_pair_no(const ConvArgs& a1, const ConvArgs& a2, hipStream_t st) {
+  switch ((a1.cout + 15) / 16) {
+    case 1: return launch_pair<XM, 1>(a1, a2, st);
+    case 2: return launch_pair<XM, 2>(a1, a2, st);
+    case 3: return launch_pair<XM, 3>(a1, a2, st);
+    default: return launch_pair<XM, 6>(a1, a2, st);
+  }
+}
+
 template <int XM, int NT, int HMAX>
 int launch_no(const ConvArgs& a, int no, hipStream_t st) {
   switch (no) {
@@ -1139,6 +1398,31 @@ extern "C" int gsvk_conv1d(int dtype, int round_x, const void* x, size_t ldx,
 namespace gsvk {
 
 bool conv1d_group_pays(size_t C, size_t T) { return (T + 63) / 64 * ((C + 31) / 32) <= 200; }
+
+int conv1d_pair(int dtype, int round_x, const ConvItem& c1, const ConvItem& c2, float slope, size_t ld,
+                size_t C, size_t T, void* stream) {
+  // each half checked with the pair's own ends: t_a is in no buffer
+  ConvArgs a1, a2;
+  if (int rc = conv1d_args(a1, c1.x, ld, c1.w_packed, c1.bias, GSVK_CONV_EPI_LRELU | GSVK_CONV_X_LRELU,
+                           slope, nullptr, nullptr, ld, c2.cur, ld, C, C, T, c1.k, c1.dilation))
+    return rc;
+  if (int rc = conv1d_args(a2, c1.x, ld, c2.w_packed, c2.bias, GSVK_CONV_EPI_RES, slope, c2.cur,
+                           c2.res, ld, nullptr, ld, C, C, T, c2.k, c2.dilation))
+    return rc;
+  if (c1.k != c2.k || c2.dilation != 1 ||
+      !conv1d_pair_fits(C, T, c1.k, c1.dilation, dtype_size(dtype)))
+    return GSVK_E_ARG;
+  if (int rc = conv_check(a1, dtype, T, T, gsvk_conv1d_packed_elems(C, C, c1.k) * 2)) return rc;
+  if (int rc = conv_check(a2, dtype, T, T, gsvk_conv1d_packed_elems(C, C, c2.k) * 2)) return rc;
+  if (!a2.res) return GSVK_E_ALIAS;  // in place: other workgroups still read the columns
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == GSVK_F16) return launch_pair_no<kXF16>(a1, a2, st);
+  return round_x ? launch_pair_no<kXRound>(a1, a2, st) : launch_pair_no<kXSplit>(a1, a2, st);
+}
+
+bool conv1d_pair_fits(size_t C, size_t T, size_t k, size_t dilation, size_t esz) {
+  return (C <= 48 || (C > 80 && C <= 96 && T >= 8192)) && C % 8 == 0 && k <= 17 && (k - 1) * dilation <= 64 && C * T * esz < (1ul << 31);
+}
 
 int conv1d_group(int dtype, int round_x, const ConvItem* items, int n, int epi, float slope,
                  size_t ld, size_t C, size_t T, void* stream) {

@@ -136,9 +136,22 @@ int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_
       // cur_j = res + convs2[m](t_a)  (dec.hpp:325-326)
       c2[m][i] = {ta, S.w2[j][m], S.b2[j][m], cur, src, nullptr, S.res_k[j], 1};
     }
+  // Narrow stages run a pair as one launch, from one buffer into another: y -> cur -> t_a -> cur.
+  bool pairs = true;
+  for (size_t j = 0; j < GSVK_SOVITS_RESBLOCKS; ++j)
+    for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m)
+      pairs = pairs && gsvk::conv1d_pair_fits(C, T, S.res_k[j], S.res_dil[m], dt == GSVK_F32 ? 4 : 2);
   // The convolutions of ResBlocks i .. i + n - 1 (in that order) on stream bst.
   auto blocks = [&](size_t i, int n, void* bst) -> int {
     for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m) {
+      if (pairs && n == 1) {
+        const size_t j = ord[i];
+        gsvk::ConvItem p1 = c1[m][i], p2 = c2[m][i];
+        p1.x = p2.res = m == 0 ? buf[kY] : m == 1 ? buf[kCur0 + j] : buf[kTa0 + j];
+        p2.cur = m == 1 ? buf[kTa0 + j] : buf[kCur0 + j];
+        if (int e = gsvk::conv1d_pair(dt, rx, p1, p2, slope, T, C, T, bst)) return e;
+        continue;
+      }
       if (int e = gsvk::conv1d_group(dt, rx, &c1[m][i], n,
                                      GSVK_CONV_EPI_LRELU | GSVK_CONV_X_LRELU, slope, T, C, T,
                                      bst))
@@ -149,6 +162,7 @@ int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_
     }
     return GSVK_OK;
   };
+  static_assert(GSVK_SOVITS_PAIRS == 3, "the buffers the pairs alternate between");
   if (gsvk::conv1d_group_pays(C, T)) {
     if (int rc = blocks(0, GSVK_SOVITS_RESBLOCKS, st)) return rc;
   } else if (!br) {

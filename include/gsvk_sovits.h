@@ -80,7 +80,8 @@ size_t gsvk_sovits_decoder_workspace_bytes(const gsvk_sovits_decoder_desc* desc)
  * Two ResBlocks of each stage run on two streams the library keeps per device, ordered after
  * the work already on `stream` and joined back into it (each stage's branch mean waits for them), so
  * `stream` orders the whole decoder as usual; a stage of few columns (up to 200 tiles of 64 columns x
- * 32 channels) runs the three ResBlocks' m-th convolutions as one launch on `stream` instead. Those streams are created on the device's first call:
+ * 32 channels) runs the three ResBlocks' m-th convolutions as one launch on `stream` instead, and a
+ * wider one of up to 48 channels (96 from 8192 columns) each pair of convolutions as one. Those streams are created on the device's first call:
  * a caller recording this call into a graph of its own makes one call outside the capture first
  * (gsvk_sovits_decoder_create records the same launches by itself). */
 int gsvk_sovits_decoder_eager(const gsvk_sovits_decoder_desc* desc, void* stream);

@@ -63,11 +63,14 @@ def test_upsampler_phases(dt, cin, cout, T, k, u):
 
 @pytest.mark.parametrize("dt,rx", [(F32, False), (F32, True), (F16, False)])
 @pytest.mark.parametrize("cin,C,T,k_up,u", [(64, 32, 9, 16, 8), (48, 24, 150, 2, 2),
-                                             (20, 20, 30, 4, 2)])
+                                             (20, 20, 30, 4, 2), (16, 24, 25703, 2, 2),
+                                             (16, 48, 13001, 2, 2), (8, 96, 8700, 2, 2),
+                                             (8, 8, 52000, 1, 1), (8, 40, 26011, 1, 1)])
 def test_stage_equals_its_convolutions(dt, rx, cin, C, T, k_up, u):
-    """gsvk.GeneratorStage (one call, grouped launches) against the same passes one by one. (20
-    channels: not for the few-tiles kernel.) Few tiles: a group and a single convolution take the same
-    tiling here, so the bits agree."""
+    """gsvk.GeneratorStage (one call: grouped launches, or pairs of convolutions in one) against the
+    same passes one by one. (20 channels: not for the few-tiles kernel.) The sizes are such that both
+    forms add in the same order: few tiles (a group and a single convolution take the same tiling), or
+    more than the few-tiles line (a pair adds as the large kernel does), so the bits agree."""
     r = rng(990 + C)
     up, rbs = make_stage(r, cin, C, k_up, u)
     st = gpu_stage(up, rbs, u)
