@@ -976,13 +976,11 @@ constexpr int kPairCols = kWaves * 32;
 constexpr int kPairTa = kPairCols + 16;  // columns of t_a in LDS: the taps of the last outputs
 
 template <int XM, int NO, int D>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(NO > 3 ? 2 : 4))) void conv_pair(PairArgs p) {
+__device__ __forceinline__ void pair_tile(const PairArgs& p, _Float16* xs) {
   constexpr int DT = storage_dt<XM>();
   constexpr int P = planes<XM>();
   constexpr int NT = 2;
   constexpr int ESZ = DT == GSVK_F32 ? 4 : 2;
-  extern __shared__ __attribute__((aligned(16))) _Float16 xs[];
   const ConvArgs& a = p.a1;
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -1177,33 +1175,64 @@ __attribute__((amdgpu_waves_per_eu(NO > 3 ? 2 : 4))) void conv_pair(PairArgs p) 
 }
 
 template <int XM, int NO>
-int launch_pair(const ConvArgs& a1, const ConvArgs& a2, hipStream_t st) {
-  auto kern = conv_pair<XM, NO, 2>;
-  PairArgs p{};
-  p.a1 = a1, p.a2 = a2;
-  p.tth = (kPairCols + a1.halo + 15) / 16 * 16;
-  p.tth_inv = static_cast<uint32_t>(((1ull << 32) + p.tth - 1) / p.tth);
-  p.out_cols = (kPairCols - (a1.k - 1)) / 4 * 4;
-  p.esz_row = static_cast<int>(a1.ldx) * (storage_dt<XM>() == GSVK_F32 ? 4 : 2);
-  const size_t lds = static_cast<size_t>(planes<XM>()) * a1.nch * 4 * std::max(p.tth, kPairTa) * 16;
-  if constexpr (NO > 3) {
-    static std::atomic<bool> lds_ok[kMaxDevices];
-    if (!allow_dynamic_lds(reinterpret_cast<const void*>(kern), 96 * 1024, lds_ok)) return GSVK_E_HIP;
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(NO > 3 ? 2 : 4))) void conv_pair(PairArgs p) {
+  extern __shared__ __attribute__((aligned(16))) _Float16 xs[];
+  pair_tile<XM, NO, 2>(p, xs);
+}
+
+// The three ResBlocks' m-th pairs side by side (grid y), as conv1d_ksplit's groups.
+struct PairGroup {
+  PairArgs p[kConvGroupMax];
+};
+template <int XM, int NO>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(NO > 3 ? 2 : 4))) void conv_pair_group(PairGroup g) {
+  extern __shared__ __attribute__((aligned(16))) _Float16 xs[];
+  pair_tile<XM, NO, 2>(g.p[blockIdx.y], xs);
+}
+
+template <int XM, int NO>
+int launch_pair(const ConvArgs* a1, const ConvArgs* a2, int n, hipStream_t st) {
+  PairGroup g{};
+  size_t lds = 0;
+  long gx = 0;
+  for (int j = 0; j < n; ++j) {
+    PairArgs& p = g.p[j];
+    p.a1 = a1[j], p.a2 = a2[j];
+    p.tth = (kPairCols + a1[j].halo + 15) / 16 * 16;
+    p.tth_inv = static_cast<uint32_t>(((1ull << 32) + p.tth - 1) / p.tth);
+    p.out_cols = (kPairCols - (a1[j].k - 1)) / 4 * 4;
+    p.esz_row = static_cast<int>(a1[j].ldx) * (storage_dt<XM>() == GSVK_F32 ? 4 : 2);
+    lds = std::max(lds, static_cast<size_t>(planes<XM>()) * a1[j].nch * 4 *
+                            std::max(p.tth, kPairTa) * 16);
+    gx = std::max(gx, (a1[j].T + p.out_cols - 1) / p.out_cols);
   }
-  const long gx = (a1.T + p.out_cols - 1) / p.out_cols;
-  p.a1.xspan = gx >= kXcdMinTiles ? (gx + kXcds - 1) / kXcds : 0;
-  const long gxl = p.a1.xspan ? p.a1.xspan * kXcds : gx;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(gxl)), dim3(kThreads), lds, st, p);
+  const long xspan = gx >= kXcdMinTiles ? (gx + kXcds - 1) / kXcds : 0;
+  for (int j = 0; j < n; ++j) g.p[j].a1.xspan = xspan;
+  const unsigned gxl = static_cast<unsigned>(xspan ? xspan * kXcds : gx);
+  constexpr size_t kMaxLds = 96 * 1024;
+  const void* kern = n == 1 ? reinterpret_cast<const void*>(conv_pair<XM, NO>)
+                            : reinterpret_cast<const void*>(conv_pair_group<XM, NO>);
+  if constexpr (NO > 3) {
+    static std::atomic<bool> lds_ok[2][kMaxDevices];
+    if (!allow_dynamic_lds(kern, kMaxLds, lds_ok[n == 1])) return GSVK_E_HIP;
+  }
+  if (n == 1)
+    hipLaunchKernelGGL((conv_pair<XM, NO>), dim3(gxl), dim3(kThreads), lds, st, g.p[0]);
+  else
+    hipLaunchKernelGGL((conv_pair_group<XM, NO>), dim3(gxl, static_cast<unsigned>(n)),
+                       dim3(kThreads), lds, st, g);
   return launch_status();
 }
 
 template <int XM>
-int launch_pair_no(const ConvArgs& a1, const ConvArgs& a2, hipStream_t st) {
-  switch ((a1.cout + 15) / 16) {
-    case 1: return launch_pair<XM, 1>(a1, a2, st);
-    case 2: return launch_pair<XM, 2>(a1, a2, st);
-    case 3: return launch_pair<XM, 3>(a1, a2, st);
-    default: return launch_pair<XM, 6>(a1, a2, st);
+int launch_pair_no(const ConvArgs* a1, const ConvArgs* a2, int n, hipStream_t st) {
+  switch ((a1->cout + 15) / 16) {
+    case 1: return launch_pair<XM, 1>(a1, a2, n, st);
+    case 2: return launch_pair<XM, 2>(a1, a2, n, st);
+    case 3: return launch_pair<XM, 3>(a1, a2, n, st);
+    default: return launch_pair<XM, 6>(a1, a2, n, st);
   }
 }
 
@@ -1399,25 +1428,29 @@ namespace gsvk {
 
 bool conv1d_group_pays(size_t C, size_t T) { return (T + 63) / 64 * ((C + 31) / 32) <= 200; }
 
-int conv1d_pair(int dtype, int round_x, const ConvItem& c1, const ConvItem& c2, float slope, size_t ld,
-                size_t C, size_t T, void* stream) {
-  // each half checked with the pair's own ends: t_a is in no buffer
-  ConvArgs a1, a2;
-  if (int rc = conv1d_args(a1, c1.x, ld, c1.w_packed, c1.bias, GSVK_CONV_EPI_LRELU | GSVK_CONV_X_LRELU,
-                           slope, nullptr, nullptr, ld, c2.cur, ld, C, C, T, c1.k, c1.dilation))
-    return rc;
-  if (int rc = conv1d_args(a2, c1.x, ld, c2.w_packed, c2.bias, GSVK_CONV_EPI_RES, slope, c2.cur,
-                           c2.res, ld, nullptr, ld, C, C, T, c2.k, c2.dilation))
-    return rc;
-  if (c1.k != c2.k || c2.dilation != 1 ||
-      !conv1d_pair_fits(C, T, c1.k, c1.dilation, dtype_size(dtype)))
-    return GSVK_E_ARG;
-  if (int rc = conv_check(a1, dtype, T, T, gsvk_conv1d_packed_elems(C, C, c1.k) * 2)) return rc;
-  if (int rc = conv_check(a2, dtype, T, T, gsvk_conv1d_packed_elems(C, C, c2.k) * 2)) return rc;
-  if (!a2.res) return GSVK_E_ALIAS;  // in place: other workgroups still read the columns
+int conv1d_pairs(int dtype, int round_x, const ConvItem* c1, const ConvItem* c2, int n, float slope,
+                 size_t ld, size_t C, size_t T, void* stream) {
+  if (n < 1 || n > kConvGroupMax) return GSVK_E_SIZE;
+  ConvArgs a1[kConvGroupMax], a2[kConvGroupMax];
+  for (int j = 0; j < n; ++j) {
+    // each half checked with the pair's own ends: t_a is in no buffer
+    const ConvItem &p = c1[j], &q = c2[j];
+    if (int rc = conv1d_args(a1[j], p.x, ld, p.w_packed, p.bias,
+                             GSVK_CONV_EPI_LRELU | GSVK_CONV_X_LRELU, slope, nullptr, nullptr, ld,
+                             q.cur, ld, C, C, T, p.k, p.dilation))
+      return rc;
+    if (int rc = conv1d_args(a2[j], p.x, ld, q.w_packed, q.bias, GSVK_CONV_EPI_RES, slope, q.cur,
+                             q.res, ld, nullptr, ld, C, C, T, q.k, q.dilation))
+      return rc;
+    if (p.k != q.k || q.dilation != 1 || !conv1d_pair_fits(C, T, p.k, p.dilation, dtype_size(dtype)))
+      return GSVK_E_ARG;
+    if (int rc = conv_check(a1[j], dtype, T, T, gsvk_conv1d_packed_elems(C, C, p.k) * 2)) return rc;
+    if (int rc = conv_check(a2[j], dtype, T, T, gsvk_conv1d_packed_elems(C, C, q.k) * 2)) return rc;
+    if (!a2[j].res) return GSVK_E_ALIAS;  // in place: other workgroups still read the columns
+  }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == GSVK_F16) return launch_pair_no<kXF16>(a1, a2, st);
-  return round_x ? launch_pair_no<kXRound>(a1, a2, st) : launch_pair_no<kXSplit>(a1, a2, st);
+  if (dtype == GSVK_F16) return launch_pair_no<kXF16>(a1, a2, n, st);
+  return round_x ? launch_pair_no<kXRound>(a1, a2, n, st) : launch_pair_no<kXSplit>(a1, a2, n, st);
 }
 
 bool conv1d_pair_fits(size_t C, size_t T, size_t k, size_t dilation, size_t esz) {

@@ -35,13 +35,13 @@ bool conv1d_group_pays(size_t C, size_t T);
 int conv1d_group(int dtype, int round_x, const ConvItem* items, int n, int epi, float slope,
                  size_t ld, size_t C, size_t T, void* stream);
 
-// A ResBlock pair, c2.cur = c2.res + conv2(lrelu(conv1(lrelu(c1.x)))) (c1.y, c1.cur, c2.x, c2.y not
-// used), in one launch, for shapes conv1d_pair_fits takes (both convolutions of one k, the second of
-// dilation 1; rows of stride T at most 2^31 bytes in all). c2.cur must not overlap c1.x or c2.res:
-// other workgroups still read their columns.
+// n ResBlock pairs, c2[j].cur = c2[j].res + conv2(lrelu(conv1(lrelu(c1[j].x)))) (c1.y, c1.cur, c2.x,
+// c2.y not used), in one launch, for shapes conv1d_pair_fits takes (both convolutions of a pair of one
+// k, the second of dilation 1; rows of stride T at most 2^31 bytes in all). c2.cur must not overlap
+// c1.x or c2.res: other workgroups still read their columns. List the longest first.
 bool conv1d_pair_fits(size_t C, size_t T, size_t k, size_t dilation, size_t esz);
-int conv1d_pair(int dtype, int round_x, const ConvItem& c1, const ConvItem& c2, float slope, size_t ld,
-                size_t C, size_t T, void* stream);
+int conv1d_pairs(int dtype, int round_x, const ConvItem* c1, const ConvItem* c2, int n, float slope,
+                 size_t ld, size_t C, size_t T, void* stream);
 
 }  // namespace gsvk
 

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <mutex>
+#include <vector>
 
 #include "gsvk.h"
 #include "gsvk_conv_group.hpp"
@@ -104,11 +105,21 @@ int count_launches(const gsvk_sovits_decoder_desc* d) {
   return (d->g_in ? 1 : 0) + 1 + 20 * static_cast<int>(d->n_stages) + 1;
 }
 
+// Where the pairs of the three ResBlocks share a launch instead of running on branches. A recorded
+// graph: the branches' fork and join cost about 20 us a stage, but a branch runs into its next pair
+// while another's last workgroups drain. Whole decoder, us, branches against shared up to 1.2 M / 2.4 M
+// elements: 75 frames fp16 586 / 565 / 568, exact 744 / 725 / 733, 150 frames 757 / 751 / 770 and 966 /
+// 967 / 987. Issued eagerly the branches also cost host calls and cross-stream waits. One stage, us:
+// 96 x 16006 exact 244 -> 166, 24 x 40000 117 -> 66, 24 x 120000 171 -> 139 (level above 5 M).
+constexpr size_t kTogetherGraph = 1200000, kTogetherEager = 5000000;
+
 // One Generator stage (dec.hpp:283-336): out = lrelu(mean_j ResBlock_j(ups(x)), slope_next). x
 // [c_in, T] with row stride ldx arrives LeakyReLU'd; buf[kY .. kSlots - 1] hold c_out x T ups_u
-// elements each. br: the streams ResBlocks 1 and 2 may run on (nullptr: all on st).
+// elements each. br: the streams ResBlocks 1 and 2 may run on (nullptr: all on st). together: the
+// three ResBlocks' m-th pairs share a launch up to this many elements of one activation.
 int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_t ldx, size_t T,
-                void* const* buf, float slope_next, void* out, void* st, const Branches* br) {
+                void* const* buf, float slope_next, void* out, void* st, const Branches* br,
+                size_t together) {
   const float slope = 0.1f;  // LRELU_SLOPE (dec.hpp:284, 322, 324)
   const size_t C = S.c_out, Tu = T * S.ups_u;
   // y = ups(x)  (dec.hpp:285)
@@ -137,19 +148,23 @@ int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_
       c2[m][i] = {ta, S.w2[j][m], S.b2[j][m], cur, src, nullptr, S.res_k[j], 1};
     }
   // Narrow stages run a pair as one launch, from one buffer into another: y -> cur -> t_a -> cur.
-  bool pairs = true;
+  const bool grouped = gsvk::conv1d_group_pays(C, T);
+  bool pairs = !grouped;
   for (size_t j = 0; j < GSVK_SOVITS_RESBLOCKS; ++j)
     for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m)
       pairs = pairs && gsvk::conv1d_pair_fits(C, T, S.res_k[j], S.res_dil[m], dt == GSVK_F32 ? 4 : 2);
   // The convolutions of ResBlocks i .. i + n - 1 (in that order) on stream bst.
   auto blocks = [&](size_t i, int n, void* bst) -> int {
     for (size_t m = 0; m < GSVK_SOVITS_PAIRS; ++m) {
-      if (pairs && n == 1) {
-        const size_t j = ord[i];
-        gsvk::ConvItem p1 = c1[m][i], p2 = c2[m][i];
-        p1.x = p2.res = m == 0 ? buf[kY] : m == 1 ? buf[kCur0 + j] : buf[kTa0 + j];
-        p2.cur = m == 1 ? buf[kTa0 + j] : buf[kCur0 + j];
-        if (int e = gsvk::conv1d_pair(dt, rx, p1, p2, slope, T, C, T, bst)) return e;
+      if (pairs) {
+        gsvk::ConvItem p1[GSVK_SOVITS_RESBLOCKS], p2[GSVK_SOVITS_RESBLOCKS];
+        for (int e = 0; e < n; ++e) {
+          const size_t j = ord[i + e];
+          p1[e] = c1[m][i + e], p2[e] = c2[m][i + e];
+          p1[e].x = p2[e].res = m == 0 ? buf[kY] : m == 1 ? buf[kCur0 + j] : buf[kTa0 + j];
+          p2[e].cur = m == 1 ? buf[kTa0 + j] : buf[kCur0 + j];
+        }
+        if (int e = gsvk::conv1d_pairs(dt, rx, p1, p2, n, slope, T, C, T, bst)) return e;
         continue;
       }
       if (int e = gsvk::conv1d_group(dt, rx, &c1[m][i], n,
@@ -163,7 +178,7 @@ int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_
     return GSVK_OK;
   };
   static_assert(GSVK_SOVITS_PAIRS == 3, "the buffers the pairs alternate between");
-  if (gsvk::conv1d_group_pays(C, T)) {
+  if (grouped || (pairs && C * T <= together)) {
     if (int rc = blocks(0, GSVK_SOVITS_RESBLOCKS, st)) return rc;
   } else if (!br) {
     for (size_t i = 0; i < GSVK_SOVITS_RESBLOCKS; ++i)
@@ -173,8 +188,9 @@ int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_
     if (hipEventRecord(br->fork, static_cast<hipStream_t>(st)) != hipSuccess) return GSVK_E_HIP;
     for (int i = 0; i < kSide; ++i)
       if (hipStreamWaitEvent(br->side[i], br->fork, 0) != hipSuccess) rc = GSVK_E_HIP;
-    for (size_t i = 0; i < GSVK_SOVITS_RESBLOCKS && rc == GSVK_OK; ++i)
-      rc = blocks(i, 1, i > 0 ? br->side[i - 1] : st);
+    // (the longest ResBlock last: on the main stream it measured 1-2% slower at 192 channels)
+    for (size_t i = GSVK_SOVITS_RESBLOCKS; i-- > 0 && rc == GSVK_OK;)
+      rc = blocks(i, 1, i + 1 < GSVK_SOVITS_RESBLOCKS ? br->side[kSide - 1 - i] : st);
     // every side stream joins back, also after an error (a capture must end joined)
     for (int i = 0; i < kSide; ++i)
       if ((hipEventRecord(br->join[i], br->side[i]) != hipSuccess ||
@@ -190,7 +206,8 @@ int issue_stage(int dt, int rx, const gsvk_sovits_stage& S, const void* x, size_
 }
 
 // The launches of one decoder pass in Generator::forward's order.
-int issue(const gsvk_sovits_decoder_desc* d, const Layout& lay, void* st, const Branches* br) {
+int issue(const gsvk_sovits_decoder_desc* d, const Layout& lay, void* st, const Branches* br,
+          size_t together) {
   const int dt = d->dtype, rx = d->round_x;
   const float slope = 0.1f;  // LRELU_SLOPE (dec.hpp:284, 322, 324)
   char* ws = static_cast<char*>(d->workspace);
@@ -218,7 +235,8 @@ int issue(const gsvk_sovits_decoder_desc* d, const Layout& lay, void* st, const 
 
   for (size_t s = 0; s < d->n_stages; ++s) {
     const float next_slope = s + 1 < d->n_stages ? slope : 0.01f;
-    if ((rc = issue_stage(dt, rx, d->stage[s], slot[kX], T, T, slot, next_slope, slot[kX], st, br)))
+    if ((rc = issue_stage(dt, rx, d->stage[s], slot[kX], T, T, slot, next_slope, slot[kX], st, br,
+                          together)))
       return rc;
     T *= d->stage[s].ups_u;
   }
@@ -247,6 +265,58 @@ int device_side_streams(hipStream_t (&side)[kSide]) {
     side[i] = streams[dev][i];
   }
   return GSVK_OK;
+}
+
+// The fork and join events of an eager call, kept between calls (creating and destroying three on each
+// call costs more host time than their records): taken for the issue of one call and given back after
+// it, when every wait on them has been enqueued. At most kKeptEvents sets per device are kept.
+struct EventSet {
+  hipEvent_t fork = nullptr, join[kSide] = {};
+};
+constexpr size_t kKeptEvents = 8;
+std::mutex events_mu;
+std::vector<EventSet> events[kMaxDevices];
+
+void destroy(EventSet& e) {
+  if (e.fork) (void)hipEventDestroy(e.fork);
+  for (int i = 0; i < kSide; ++i)
+    if (e.join[i]) (void)hipEventDestroy(e.join[i]);
+  e = EventSet{};
+}
+
+// Issues f(Branches) on the side streams with events of its own (fresh: none that are kept).
+template <class F>
+int with_branches(const hipStream_t* side, bool fresh, F f) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return GSVK_E_HIP;
+  EventSet e;
+  if (!fresh) {
+    std::lock_guard<std::mutex> lock(events_mu);
+    if (!events[dev].empty()) e = events[dev].back(), events[dev].pop_back();
+  }
+  int rc = GSVK_OK;
+  if (!e.fork) {
+    if (hipEventCreateWithFlags(&e.fork, hipEventDisableTiming) != hipSuccess) rc = GSVK_E_HIP;
+    for (int i = 0; i < kSide && rc == GSVK_OK; ++i)
+      if (hipEventCreateWithFlags(&e.join[i], hipEventDisableTiming) != hipSuccess) rc = GSVK_E_HIP;
+  }
+  if (rc == GSVK_OK) rc = f(Branches{side, e.fork, e.join});
+  if (rc == GSVK_OK && !fresh) {
+    std::lock_guard<std::mutex> lock(events_mu);
+    if (events[dev].size() < kKeptEvents) {
+      events[dev].push_back(e);
+      return rc;
+    }
+  }
+  destroy(e);  // (an event destroyed while its record is pending is released once that completes)
+  return rc;
+}
+
+// Whether a call on st is being captured: its events are then the capture's, and not kept.
+bool capturing(void* st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(static_cast<hipStream_t>(st), &s) != hipSuccess ||
+         s != hipStreamCaptureStatusNone;
 }
 
 }  // namespace
@@ -295,22 +365,14 @@ extern "C" int gsvk_sovits_stage_eager(int dtype, int round_x, const gsvk_sovits
   void* buf[kSlots] = {};
   for (int i = kY; i < kSlots; ++i) buf[i] = static_cast<char*>(workspace) + (i - kY) * slot;
   if (!side || gsvk::conv1d_group_pays(stage->c_out, T * stage->ups_u))
-    return issue_stage(dtype, round_x, *stage, x, ldx, T, buf, slope_next, out, stream, nullptr);
+    return issue_stage(dtype, round_x, *stage, x, ldx, T, buf, slope_next, out, stream, nullptr,
+                       kTogetherEager);
   hipStream_t sd[kSide];
-  hipEvent_t fork = nullptr, join[kSide] = {};
-  int rc = hipEventCreateWithFlags(&fork, hipEventDisableTiming) == hipSuccess ? GSVK_OK : GSVK_E_HIP;
-  for (int i = 0; i < kSide && rc == GSVK_OK; ++i) {
-    sd[i] = static_cast<hipStream_t>(side[i]);
-    if (hipEventCreateWithFlags(&join[i], hipEventDisableTiming) != hipSuccess) rc = GSVK_E_HIP;
-  }
-  if (rc == GSVK_OK) {
-    const Branches br{sd, fork, join};
-    rc = issue_stage(dtype, round_x, *stage, x, ldx, T, buf, slope_next, out, stream, &br);
-  }
-  if (fork) (void)hipEventDestroy(fork);
-  for (int i = 0; i < kSide; ++i)
-    if (join[i]) (void)hipEventDestroy(join[i]);
-  return rc;
+  for (int i = 0; i < kSide; ++i) sd[i] = static_cast<hipStream_t>(side[i]);
+  return with_branches(sd, capturing(stream), [&](const Branches& br) {
+    return issue_stage(dtype, round_x, *stage, x, ldx, T, buf, slope_next, out, stream, &br,
+                       kTogetherEager);
+  });
 }
 
 extern "C" int gsvk_sovits_decoder_eager(const gsvk_sovits_decoder_desc* desc, void* stream) {
@@ -318,21 +380,10 @@ extern "C" int gsvk_sovits_decoder_eager(const gsvk_sovits_decoder_desc* desc, v
   int rc = check_workspace(desc, &lay);
   if (rc) return rc;
   hipStream_t side[kSide];
-  hipEvent_t fork = nullptr, join[kSide] = {};
-  rc = device_side_streams(side);
-  if (rc == GSVK_OK && hipEventCreateWithFlags(&fork, hipEventDisableTiming) != hipSuccess)
-    rc = GSVK_E_HIP;
-  for (int i = 0; i < kSide && rc == GSVK_OK; ++i)
-    if (hipEventCreateWithFlags(&join[i], hipEventDisableTiming) != hipSuccess) rc = GSVK_E_HIP;
-  if (rc == GSVK_OK) {
-    const Branches br{side, fork, join};
-    rc = issue(desc, lay, stream, &br);
-  }
-  // (an event destroyed while its record is pending is released once that work completes)
-  if (fork) (void)hipEventDestroy(fork);
-  for (int i = 0; i < kSide; ++i)
-    if (join[i]) (void)hipEventDestroy(join[i]);
-  return rc;
+  if ((rc = device_side_streams(side))) return rc;
+  return with_branches(side, capturing(stream), [&](const Branches& br) {
+    return issue(desc, lay, stream, &br, kTogetherEager);
+  });
 }
 
 extern "C" int gsvk_sovits_decoder_create(const gsvk_sovits_decoder_desc* desc,
@@ -351,7 +402,7 @@ extern "C" int gsvk_sovits_decoder_create(const gsvk_sovits_decoder_desc* desc,
          const hipEvent_t* join) {
         const Ctx* x = static_cast<const Ctx*>(c);
         const Branches br{side, fork, join};
-        return issue(x->d, x->lay, st, &br);
+        return issue(x->d, x->lay, st, &br, kTogetherGraph);
       },
       &ctx, GSVK_SOVITS_RESBLOCKS - 1, count_launches(desc), out);
 }
