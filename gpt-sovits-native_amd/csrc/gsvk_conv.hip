@@ -59,7 +59,6 @@ struct ConvArgs {
   void* y;
   long cin, cout, T, ldx, ldc, ldy;  // T: input columns
   int k, dil, pad, nch, opad;
-  int halo;  // staged columns past a tile: (k - 1) dil, or ceil(k / u) - 1
   int epi;
   float slope;
   bool vec;
@@ -67,8 +66,6 @@ struct ConvArgs {
   int up;     // 0: Conv1d; u: transposed convolution with stride u (phase r = blockIdx.z)
   long Tout;  // transposed: output columns T u
   int pad_t;  // transposed: (k - u) / 2
-  int kq, kr, pq, pr, er;  // transposed: k, pad_t and Tout - 1 + pad_t divided by u (block_map)
-  long eq;
   long xspan;  // time tiles per XCD (the grid's x extent / kXcds), 0: x index = time tile
 };
 
@@ -97,27 +94,72 @@ struct Map {
   const uint16_t* wp;
 };
 
-// The phases' geometry without a division on the device (a 64-bit one costs a workgroup several
-// hundred cycles before its first load): with k = kq u + kr, pad_t = pq u + pr and
-// Tout - 1 + pad_t = eq u + er, all formed on the host, phase r < u has
-//   kn = kq + (r < kr), and the phases before it r kq + min(r, kr) taps;
-//   qlo = ceil((pad_t - r) / u) = pq + (pr > r), qhi = floor((Tout - 1 + pad_t - r) / u) =
-//   eq - (er < r).
-__device__ __forceinline__ Map block_map(const ConvArgs& a, int r) {
+__device__ __forceinline__ long ceil_div(long a, long b) { return a >= 0 ? (a + b - 1) / b : -((-a) / b); }
+__device__ __forceinline__ long floor_div(long a, long b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
+
+__device__ __forceinline__ Map block_map(const ConvArgs& a) {
   Map m;
   if (!a.up) {
     m.kn = a.k, m.nq = a.T, m.xoff = -a.pad, m.ostr = 1, m.obase = 0, m.wp = a.wp;
     return m;
   }
-  m.kn = a.kq + (r < a.kr ? 1 : 0);
-  const size_t taps_before = static_cast<size_t>(r * a.kq + min(r, a.kr));
+  const int u = a.up, r = blockIdx.z;
+  m.kn = (a.k - r + u - 1) / u;
+  size_t taps_before = 0;
+  for (int r2 = 0; r2 < r; ++r2) taps_before += static_cast<size_t>((a.k - r2 + u - 1) / u);
   m.wp = a.wp + taps_before * a.nch * a.opad * kChunk;
-  const long qlo = a.pq + (a.pr > r ? 1 : 0), qhi = a.eq - (a.er < r ? 1 : 0);
+  const long qlo = ceil_div(a.pad_t - r, u), qhi = floor_div(a.Tout - 1 + a.pad_t - r, u);
+  m.nq = qhi - qlo + 1;
+  m.xoff = qlo - (m.kn - 1);
+  m.ostr = u;
+  m.obase = qlo * u + r - a.pad_t;
+  return m;
+}
+
+// The same without a division on the device (a 64-bit one costs a short-lived workgroup several hundred
+// cycles before its first load; conv1d_mfma keeps block_map, whose other code measured the same or up
+// to 4% slower around this form). With k = kq u + kr, pad_t = pq u + pr and Tout - 1 + pad_t = eq u +
+// er, all formed on the host, phase r < u has
+//   kn = kq + (r < kr), and the phases before it r kq + min(r, kr) taps;
+//   qlo = ceil((pad_t - r) / u) = pq + (pr > r), qhi = floor((Tout - 1 + pad_t - r) / u) =
+//   eq - (er < r).
+struct Phases {
+  int kq, kr, pq, pr, er;
+  long eq;
+};
+
+__device__ __forceinline__ Map plain_map(const ConvArgs& a) {
+  Map m;
+  m.kn = a.k, m.nq = a.T, m.xoff = -a.pad, m.ostr = 1, m.obase = 0, m.wp = a.wp;
+  return m;
+}
+
+__device__ __forceinline__ Map phase_map(const ConvArgs& a, const Phases& p, int r) {
+  if (!a.up) return plain_map(a);
+  Map m;
+  m.kn = p.kq + (r < p.kr ? 1 : 0);
+  const size_t taps_before = static_cast<size_t>(r * p.kq + min(r, p.kr));
+  m.wp = a.wp + taps_before * a.nch * a.opad * kChunk;
+  const long qlo = p.pq + (p.pr > r ? 1 : 0), qhi = p.eq - (p.er < r ? 1 : 0);
   m.nq = qhi - qlo + 1;
   m.xoff = qlo - (m.kn - 1);
   m.ostr = a.up;
   m.obase = qlo * a.up + r - a.pad_t;
   return m;
+}
+
+Phases phases_of(const ConvArgs& a) {
+  Phases p{};
+  if (!a.up) return p;
+  p.kq = a.k / a.up, p.kr = a.k % a.up;
+  p.pq = a.pad_t / a.up, p.pr = a.pad_t % a.up;
+  p.eq = (a.Tout - 1 + a.pad_t) / a.up, p.er = static_cast<int>((a.Tout - 1 + a.pad_t) % a.up);
+  return p;
+}
+
+// Staged columns past a tile.
+int halo_of(const ConvArgs& a) {
+  return a.up ? (a.k + a.up - 1) / a.up - 1 : (a.k - 1) * a.dil;
 }
 
 template <int XM>
@@ -332,7 +374,7 @@ __attribute__((amdgpu_waves_per_eu(conv_waves_per_eu<XM>(FS)))) void conv1d_mfma
                : static_cast<long>(blockIdx.x)) *
       TT;
   const long o0 = static_cast<long>(blockIdx.y) * (FS * NO);
-  const Map m = block_map(a, blockIdx.z);
+  const Map m = block_map(a);
   if (t0 >= m.nq) return;  // a phase with fewer positions than the grid covers (whole workgroup)
 
   // ---- x chunk: global -> registers -> LDS ------------------------------------------------------
@@ -694,6 +736,7 @@ struct KsArgs {
   unsigned ntiles_t, ntiles_o, phases;
   unsigned span;  // tiles per XCD
   int esz_row;   // bytes of a row of x
+  Phases ph;
 };
 
 template <int XM, int NT, int NO, int KW, int D>
@@ -711,7 +754,7 @@ __device__ __forceinline__ void ksplit_tile(const ConvArgs& a, const KsArgs& ks,
   // Tiles are numbered time fastest, then output-row blocks, then phases.
   const unsigned oz = tile / ks.ntiles_t, z = oz / ks.ntiles_o;  // phase (0 without phases)
   if (z >= ks.phases) return;
-  const Map m = block_map(a, static_cast<int>(z));
+  const Map m = phase_map(a, ks.ph, static_cast<int>(z));
   const long o0 = static_cast<long>(oz - z * ks.ntiles_o) * (16 * NO);
   const long t0 = static_cast<long>(tile - oz * ks.ntiles_t) * TT;
   if (t0 >= m.nq) return;
@@ -904,7 +947,8 @@ int launch_ksplit(const ConvArgs* a, int n, hipStream_t st) {
   for (int j = 0; j < n; ++j) {
     g.a[j] = a[j];
     KsArgs& ks = g.ks[j];
-    ks.tth = (16 * NT + a[j].halo + 15) / 16 * 16;
+    ks.ph = phases_of(a[j]);
+    ks.tth = (16 * NT + halo_of(a[j]) + 15) / 16 * 16;
     ks.tth_inv = static_cast<uint32_t>(((1ull << 32) + ks.tth - 1) / ks.tth);
     const int chunk_bytes = planes<XM>() * 4 * ks.tth * 16;
     const int cb = std::max(1, kKsLds / chunk_bytes);
@@ -930,7 +974,7 @@ long ks_tiles(const ConvArgs& a) {
 // Whether conv1d_ksplit can run a: its staging loads eight channels of one column at 32-bit offsets
 // into the whole of x.
 bool ks_ok(const ConvArgs& a, size_t esz) {
-  return a.halo <= 64 && a.cout >= 24 && a.cin % 8 == 0 &&
+  return halo_of(a) <= 64 && a.cout >= 24 && a.cin % 8 == 0 &&
          static_cast<size_t>(a.cin) * a.ldx * esz < (1ul << 31);
 }
 
@@ -1151,7 +1195,7 @@ __device__ __forceinline__ void pair_tile(const PairArgs& p, _Float16* xs) {
     *reinterpret_cast<u32x4*>(xs + q * plane + (static_cast<size_t>(2 * NO) * kPairTa + r) * 8) =
         u32x4{0u, 0u, 0u, 0u};
   }
-  const Map m = block_map(p.a2, 0);
+  const Map m = plain_map(p.a2);
   f4v cur[NT][NO];
 #pragma unroll
   for (int n = 0; n < NO; ++n)
@@ -1200,7 +1244,7 @@ int launch_pair(const ConvArgs* a1, const ConvArgs* a2, int n, hipStream_t st) {
   for (int j = 0; j < n; ++j) {
     PairArgs& p = g.p[j];
     p.a1 = a1[j], p.a2 = a2[j];
-    p.tth = (kPairCols + a1[j].halo + 15) / 16 * 16;
+    p.tth = (kPairCols + halo_of(a1[j]) + 15) / 16 * 16;
     p.tth_inv = static_cast<uint32_t>(((1ull << 32) + p.tth - 1) / p.tth);
     p.out_cols = (kPairCols - (a1[j].k - 1)) / 4 * 4;
     p.esz_row = static_cast<int>(a1[j].ldx) * (storage_dt<XM>() == GSVK_F32 ? 4 : 2);
@@ -1265,7 +1309,7 @@ int launch_plan(const ConvArgs& a, hipStream_t st) {
   // Halos of up to 16 columns (k 3 at dilations up to 8, every dilation-1 ResBlock convolution,
   // the upsamplers) take the kernels with the 16-column halo slab; measured on the decoder
   // graph, 3% faster exact than staging a 64-column halo block for them.
-  const int halo = a.halo;
+  const int halo = halo_of(a);
   // Few tiles: the K-split kernel. The line was measured on the whole decoder, its ResBlocks on
   // concurrent branches, at 20 to 500 frames.
   constexpr long kKsTiles = XM == kXSplit ? 600 : 800;
@@ -1403,7 +1447,6 @@ int conv1d_args(ConvArgs& a, const void* x, size_t ldx, const uint16_t* w_packed
   a.pad = static_cast<int>((k - 1) * dilation / 2);
   a.nch = static_cast<int>((c_in + kChunk - 1) / kChunk);
   a.opad = static_cast<int>((c_out + kOPad - 1) / kOPad * kOPad);
-  a.halo = static_cast<int>((k - 1) * dilation);
   a.epi = epi, a.slope = slope;
   return GSVK_OK;
 }
@@ -1532,13 +1575,9 @@ extern "C" int gsvk_convt1d(int dtype, int round_x, const void* x, size_t ldx,
   a.k = static_cast<int>(k), a.dil = 1, a.pad = 0;
   a.nch = static_cast<int>((c_in + kChunk - 1) / kChunk);
   a.opad = static_cast<int>((c_out + kOPad - 1) / kOPad * kOPad);
-  a.halo = static_cast<int>((k + stride - 1) / stride - 1);
   a.epi = epi, a.slope = slope;
   a.up = static_cast<int>(stride), a.Tout = static_cast<long>(T * stride);
   a.pad_t = static_cast<int>((k - stride) / 2);
-  a.kq = a.k / a.up, a.kr = a.k % a.up;
-  a.pq = a.pad_t / a.up, a.pr = a.pad_t % a.up;
-  a.eq = (a.Tout - 1 + a.pad_t) / a.up, a.er = static_cast<int>((a.Tout - 1 + a.pad_t) % a.up);
   return conv_entry(a, dtype, round_x, T, T * stride,
                     gsvk_convt1d_packed_elems(c_out, c_in, k, stride) * 2,
                     static_cast<hipStream_t>(stream));
