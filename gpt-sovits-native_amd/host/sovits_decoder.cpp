@@ -21,7 +21,7 @@ size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // Workspace layout: the folded bias (c0 floats), then 8 activation slots of `slot` elements of the
 // activation dtype each: X (stage input, then the stage output), Y (upsampler output, the first
 // residual), TA0..TA2 (each ResBlock's pair middle activation, so the three ResBlocks can run
-// side by side) and CUR0..CUR2 (the three branch accumulators). The pairs' LeakyReLU inputs are
+// side by side; where a pair is one launch, the second pair's sum) and CUR0..CUR2 (the three branch accumulators). The pairs' LeakyReLU inputs are
 // not stored: the first conv of a pair reads lrelu(cur) as it loads (GSVK_CONV_X_LRELU).
 enum Slot {
   kX,
