@@ -403,6 +403,9 @@ class GeneratorStage:
 
     def forward(self, x, out, slope_next=0.1, round_x=False, stream=None):
         import torch
+        if x.is_cuda and x.device.index != torch.cuda.current_device():
+            with torch.cuda.device(x.device):  # the call's events belong to the stream's device
+                return self.forward(x, out, slope_next, round_x, stream)
         main = stream if stream is not None else torch.cuda.current_stream(x.device)
         S = self._stage()
         c_in, T, ldx = _rows(x)
