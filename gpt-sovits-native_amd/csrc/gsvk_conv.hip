@@ -979,12 +979,14 @@ bool ks_ok(const ConvArgs& a, size_t esz) {
 }
 
 // Tiles: 64 columns x 32 rows with 8 waves while all tiles of the launch run at once (two
-// workgroups per CU) and there are three units for every wave; otherwise 4 waves, on 48 rows with
-// the exact split (whose staging is twice as long) where that pads nothing.
+// workgroups per CU; a group's may run over by its short convolutions) and there are three units for
+// every wave; otherwise 4 waves, on 48 rows with the exact split (whose staging is twice as long)
+// where that pads nothing. The 564 tiles of the 192-channel stage at 75 frames with 8 waves cost the
+// whole decoder 622 -> 666 us in fp16, 768 -> 819 exact.
 template <int XM>
 int launch_ks(const ConvArgs* a, int n, hipStream_t st) {
   const int kn = (a->k + (a->up ? a->up : 1) - 1) / (a->up ? a->up : 1);
-  if (n * ks_tiles(*a) <= 600 && a->nch * kn >= 24)
+  if (n * ks_tiles(*a) <= (n > 1 ? 600 : 512) && a->nch * kn >= 24)
     return launch_ksplit<XM, 4, 2, 8, 4, 4>(a, n, st);
   if constexpr (XM == kXSplit) {
     if (a->cout >= 96 && a->cout % 48 == 0) return launch_ksplit<XM, 4, 3, 4, 4, 3>(a, n, st);
